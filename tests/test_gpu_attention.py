@@ -192,6 +192,35 @@ def test_extreme_logits_take_the_exact_path(case):
     _check(dense, OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), *dl))
 
 
+@pytest.mark.parametrize("hot", [0.0, 30.0])
+@pytest.mark.parametrize("nblk,at,reverse", [(1, 0, False), (7, 6, False), (8, 7, True), (9, 8, False), (9, 0, True),
+                                             (20, 7, False), (20, 8, True), (20, 19, False)])
+def test_range_exit_at_every_point_of_the_walk(nblk, at, reverse, hot):
+    """Block ``at`` lifts every third row's logits by about ``hot`` * 8 * log2 e
+    (above the range of exponent offset 0; hot = 0 stays inside it), before and
+    after the kernel's early look at its row sums, in lists of either order that
+    hold the partial last block, with waves that own no rows (nq = 130). Same
+    tolerance as the other extreme-logit cases: bf16 probabilities of a float64
+    softmax."""
+    from vasc_amd import ops
+    B, H, nq, nk, D = 1, 2, 130, 64 * nblk - 31, 64
+    q, k, v = (_rand((B, H, n, D), 30 + i).float() for i, n in enumerate((nq, nk, nk)))
+    u = torch.zeros(D)
+    u[:16] = 4.0 ** 0.5 / 2
+    if hot:
+        q[:, :, ::3] += hot / 4 * u
+        k[:, :, 64 * at:64 * at + 64] += 4.0 * u
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    order = np.arange(nblk)[::-1] if reverse else np.arange(nblk)
+    idx = np.ascontiguousarray(np.broadcast_to(order.astype(np.int32), (B, H, 2, nblk)))
+    cnt = np.full((B, H, 2), nblk, np.int32)
+    qc, kc, vt = q.cuda(), k.cuda(), ops.pack_v(v.cuda())
+    out = ops.block_sparse_attn(qc, kc, vt, torch.from_numpy(idx).cuda(), torch.from_numpy(cnt).cuda())
+    ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), idx, cnt)
+    _check(out, ref)
+    _check(ops.dense_attn(qc, kc, vt), ref)
+
+
 # ---------------------------------------------------------------- PV post-cut
 def _graded_blocks(nq, nk, levels, seed):
     """Query rows a*e0 (+ small noise) and key block j = levels[j] / c * e0

@@ -7,37 +7,46 @@
 // arithmetic is bf16 MFMA with fp32 accumulation instead of int8 QK^T + fp16
 // PV, and the structure is CDNA4's:
 //
-//  * 4 waves x 32 query rows. S^T = K Q^T on v_mfma_f32_32x32x16_bf16 so a
-//    lane owns one query row (lane % 32) and 32 of the 64 keys of a block.
+//  * 4 waves x 32 query rows (two tiles of 16). S^T = K Q^T on
+//    v_mfma_f32_16x16x32_bf16, so a lane owns one query row of each tile
+//    (lane % 16) and 16 of the 64 keys of a block.
+//  * The kernel runs at the card's power limit, so the clock follows what a
+//    block costs in energy: with random bf16 operands the 16x16x32 product
+//    sustains 2.23 PFLOP/s and the 32x32x16 one 1.89 (accumulators move half
+//    the register bytes per product). The change of shape took a launch over
+//    33312 keys, 16 heads and 132 blocks a row from 1.13 to 1.02 ms.
 //  * O^T = Vt P^T on the same MFMA, so P feeds the B operand straight from
-//    the S^T accumulators. Vt comes from vasc_pack_v with keys permuted into
-//    exactly the order the accumulators hold them.
-//  * The kernel is held to 128 VGPRs so four waves share each SIMD: one
-//    wave's MFMAs overlap other waves' exponentials (on gfx950 a v_exp_f32
-//    costs about 2.3 FMA issue slots; at head_dim 64 the exponentials cost
-//    as much VALU time as the MFMAs take).
-//  * The exponent offset m only has to keep probabilities inside fp32/bf16
-//    range, not equal the row max: softmax is invariant to it. m starts at
-//    0 and the fast path is P = exp2(fma(S, sm_scale*log2(e), -m)) on the
-//    exact fp32 logits: no max, no rescale. Each lane sums its block's bf16
-//    probabilities with v_dot2 (the sum is also the normaliser); a block sum
-//    above 2^64, or a running sum below 2^-60 (a row whose logits are all far
-//    below 0), sends the wave through an exact path that moves m to the row
-//    max and rescales O and the sum. The same path masks the keys of the
-//    partial last block and of blocks outside the sequence.
+//    the S^T accumulators. Vt comes from vasc_pack_v with its keys permuted;
+//    row i of S^T tile u of a 32-key group is key 8 u + 16 (i / 8) + i % 8 of
+//    the group, which puts the probabilities in exactly that order.
+//  * Row sums are products too: a ones operand against P, 4 of the block's 36
+//    MFMAs. v_dot2 (the former row sum) shares the matrix pipe: 16 of them
+//    beside 16 MFMAs and the exponentials cost a wave-block 350 cycles, the
+//    products 47 (probe without memory, four waves per SIMD).
+//  * The kernel is held to 128 VGPRs so four waves share each SIMD: MFMAs of
+//    one wave overlap the exponentials of the others (about 770 cycles per
+//    wave-block: 576 of MFMA, 450 of VALU). Two waves of 64 rows per SIMD
+//    halve the LDS reads but took 980 cycles (exposed latencies).
+//  * Softmax is invariant to the exponent offset, which only has to keep the
+//    probabilities inside fp32/bf16 range. The walk uses offset 0:
+//    P = exp2(c S) on the exact fp32 logits, no max, no rescale, no branch.
+//    A row sum outside [2^-90, 2^120] (checked after eight
+//    blocks and at the end) sends the workgroup through a second walk with
+//    the running row max as the offset, which also takes blocks outside the
+//    sequence. Checking and rescaling per block cost 2 % of the launch.
+//  * Keys past the sequence end (the partial last block) read the last key's
+//    row: their V rows are zero and the ones operand is zeroed there.
 //  * K and Vt tiles arrive by LDS DMA (global_load_lds_dwordx4) into a
-//    double-buffered LDS tile one block ahead of the MFMAs, with a
-//    16-byte-chunk xor swizzle ((row/2)%8) that spreads the rows an MFMA
-//    operand read touches over all LDS banks. The DMA is issued through asm
-//    without a memory clobber (the explicit waits and barriers order it), so
-//    the compiler neither drains it before LDS reads nor turns the uniform
-//    list reads into vector loads: the lists are read through the constant
-//    address space on the scalar unit, and nothing but the DMA counts in
-//    vmcnt inside the loop. Q is consumed before the loop so that its load
-//    wait stays out of the loop body.
-//  * The loop body runs two blocks per trip (buffers 0 and 1), so every LDS
-//    operand address is a lane constant plus an immediate offset; all eight K
-//    (and Vt) operand reads of a block are issued before its first product.
+//    double-buffered LDS tile one block ahead of the MFMAs. The 16-byte
+//    chunks of a row are xor-swizzled so that the 16 rows of an operand read
+//    fill all LDS banks: by (row/2)%8 in Vt; K operand rows are 0-7 and
+//    16-23 (8-15, 24-31) of a group, so row bit 4 replaces bit 3 there. The
+//    DMA is issued through asm without a memory clobber (the explicit waits
+//    and barriers order it), so the compiler neither drains it before LDS
+//    reads nor turns the uniform list reads into vector loads: the lists are
+//    read through the constant address space on the scalar unit, and nothing
+//    but the DMA counts in vmcnt inside the loop. Q is consumed before the
+//    loop so that its load wait stays out of the loop body.
 //  * workgroup ids are remapped so each XCD walks a contiguous range of
 //    query blocks of the same head (K/V reuse in that XCD's L2).
 //  * vasc_global_attn_fwd adds the layer's special-token queries, which
@@ -47,6 +56,8 @@
 //    workgroup), and they are remapped like the patch workgroups, so each
 //    XCD takes the special queries of the heads whose patch queries it
 //    walks and reads their K and V through the same L2.
+#include <type_traits>
+
 #include "common.h"
 
 namespace vasc {
@@ -86,7 +97,7 @@ struct AttnParams {
   // eight heads, one per XCD, would overflow the Infinity Cache); 0: each
   // XCD walks a contiguous range of query blocks
   int32_t head_major;
-  // PV post-cut (kPv instances): per-head thresholds in log2 units and the
+  // PV post-cut: per-head thresholds in log2 units and the
   // per-wave execution map [B, H, nqb * 4, pv_w] (written where PV ran)
   const float *pv_thr;
   int32_t *pv_map;
@@ -112,6 +123,11 @@ __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 // below m that they lose precision).
 constexpr float kHigh = 18446744073709551616.0f;  // 2^64
 constexpr float kLow = 8.673617379884035e-19f;    // 2^-60
+// Row sums at exponent offset 0 are good in [2^-90, 2^120]: below, flushed
+// probabilities (under 2^-126) could add up to more than 2^-23 of the sum;
+// above, the largest ones near overflow. The accumulated outputs are checked
+// for finiteness beside them.
+constexpr uint32_t kHighBits = 0x7b800000u, kLowBits = 0x12800000u;
 
 // LDS DMA without a memory clobber (the waits and barriers that order it are
 // explicit); uniform list reads then stay on the scalar unit.
@@ -123,13 +139,199 @@ __device__ __forceinline__ void dma16(const void *sbase, uint32_t voff_bytes, ui
       : "s"(lds_addr), "v"(voff_bytes), "s"(sbase));
 }
 
-template <bool kDense, bool kPv = false>
+__device__ __forceinline__ floatx4 mfma16(u32x4 a, u32x4 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// LDS chunk swizzle of K tile row r in bsattn_fwd_kernel (see above).
+__device__ __forceinline__ int swz_k(int r) { return ((r >> 1) & 3) | ((r >> 2) & 4); }
+
+constexpr int kCheckAt = 8;  // blocks walked before the first look at the row sums
+
+typedef const __attribute__((address_space(4))) AttnParams ConstParams;
+
+// Normalised results of a wave's two query tiles; a row without any
+// probability is zero. sp: the special-query outputs.
+template <typename Params>
+__device__ __forceinline__ void store_rows(const Params &p, bool sp, int64_t b, int64_t h, int64_t row0, int64_t nq,
+                                           int lr, int g4, const floatx4 (&oacc)[2][4], const floatx4 (&lacc)[2]) {
+  uint16_t *odst = sp ? p.o2 + b * p.o2_sb + h * p.o2_sh : p.o + b * p.o_sb + h * p.o_sh;
+  const int64_t o_st = sp ? p.o2_st : p.o_st;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int64_t qrow = row0 + 16 * i + lr;
+    if (qrow >= nq) continue;
+    int64_t orow = qrow;
+    if (p.tok_p > 0) {
+      const int64_t per = sp ? p.tok_s : p.tok_p - p.tok_s;  // queries per frame of this kind
+      orow = (orow / per) * p.tok_p + (sp ? 0 : p.tok_s) + orow % per;
+    }
+    uint16_t *optr = odst + orow * o_st;
+    const float ltot = lacc[i][0];
+    const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      uint2 v;
+      v.x = pack_bf16x2(oacc[i][t][0] * inv, oacc[i][t][1] * inv);
+      v.y = pack_bf16x2(oacc[i][t][2] * inv, oacc[i][t][3] * inv);
+      *reinterpret_cast<uint2 *>(optr + 16 * t + 4 * g4) = v;
+    }
+  }
+}
+
+// The workgroup of bsattn_fwd_kernel again with the running row max as the
+// exponent offset (online softmax), for rows whose sums at offset 0 left the
+// range and for lists that name blocks outside the sequence. Out of line, so
+// that the kernel's registers go to its own loop.
+__device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_arg, bool every_block, int wg_arg,
+                                           int n_arg) {
+  // the arguments arrive in VGPRs: back to scalars, and the parameters through
+  // the constant address space
+  auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); };
+  const uint64_t pa = reinterpret_cast<uint64_t>(pp);
+  const ConstParams &p = *reinterpret_cast<const ConstParams *>(
+      (static_cast<uint64_t>(uniform(static_cast<uint32_t>(pa >> 32))) << 32) | uniform(static_cast<uint32_t>(pa)));
+  const uint32_t lds0 = uniform(lds0_arg);
+  const int wg = static_cast<int>(uniform(static_cast<uint32_t>(wg_arg)));
+  const int n = static_cast<int>(uniform(static_cast<uint32_t>(n_arg)));
+  const bool dense = every_block || static_cast<int64_t>(blockIdx.x) < p.num_wg2_slots;
+  const bool sp = dense && !every_block;
+  const int64_t nqb = sp ? p.nq2b : p.nqb;
+  const int qb = static_cast<int>(wg % nqb);
+  const int64_t bh = wg / nqb, h = bh % p.H, b = bh / p.H;
+  const int tid = threadIdx.x, l = tid & 63, lr = l & 15, g4 = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  typedef const __attribute__((address_space(4))) int32_t *list_ptr;
+  const list_ptr list = (list_ptr)(dense ? nullptr : p.idx + (bh * p.nqb + qb) * p.idx_w);
+  const uint16_t *qsrc = sp ? p.q2 + b * p.q2_sb + h * p.q2_sh : p.q + b * p.q_sb + h * p.q_sh;
+  const int64_t q_st = sp ? p.q2_st : p.q_st, nq = sp ? p.nq2 : p.nq;
+  const int64_t row0 = static_cast<int64_t>(qb) * kBlockQ + w * 32;
+  const uint16_t *kbase = p.k + b * p.k_sb + h * p.k_sh;
+  const uint16_t *vbase = p.vt + bh * p.nkb * kTile;
+  typedef __attribute__((address_space(3))) u32x4 *lds_ptr;
+  u32x4 qf[2][2];
+  for (int i = 0; i < 2; ++i) {
+    const int64_t qrow = row0 + 16 * i + lr;
+    for (int s = 0; s < 2; ++s)
+      qf[i][s] = qrow < nq ? *reinterpret_cast<const u32x4 *>(qsrc + qrow * q_st + 32 * s + 8 * g4) : u32x4{0, 0, 0, 0};
+  }
+  const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+  floatx4 oacc[2][4], lacc[2];
+  float m[2];
+  for (int i = 0; i < 2; ++i) {
+    lacc[i] = zero4;
+    m[i] = -INFINITY;
+    for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
+  }
+  // the next block's chunks wait in registers while this one is computed
+  u32x4 kr[2], vr[2];
+  int j = 0, blk = 0;
+  auto next = [&]() -> int {  // the list's next block inside the sequence, -1 at its end
+    while (j < n) {
+      blk = dense ? j : (p.delta ? blk + list[j] : list[j]);
+      ++j;
+      if (blk >= 0 && blk < p.nkb) return blk;
+    }
+    return -1;
+  };
+  auto keys_of = [&](int at) {
+    const int64_t left = p.nk - static_cast<int64_t>(at) * kBlockK;
+    return static_cast<int>(left < kBlockK ? left : kBlockK);
+  };
+  auto load = [&](int at) {
+    const int last = keys_of(at) - 1;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int ci = tid + kThreads * u, r = ci >> 3, ch = ci & 7;
+      kr[u] = *reinterpret_cast<const u32x4 *>(
+          kbase + (static_cast<int64_t>(at) * kBlockK + (r < last ? r : last)) * p.k_st + ch * 8);
+      vr[u] = *reinterpret_cast<const u32x4 *>(vbase + static_cast<int64_t>(at) * kTile + ci * 8);
+    }
+  };
+  int nxt = next();
+  if (nxt >= 0) load(nxt);
+  while (nxt >= 0) {
+    const int lim = keys_of(nxt);
+    __syncthreads();  // the previous block's reads are done
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int ci = tid + kThreads * u;
+      const int at = ((ci & ~7) | ((ci & 7) ^ swz(ci >> 3))) * 16;
+      *reinterpret_cast<lds_ptr>(lds0 + at) = kr[u];
+      *reinterpret_cast<lds_ptr>(lds0 + kTile * 2 + at) = vr[u];
+    }
+    nxt = next();
+    if (nxt >= 0) load(nxt);
+    __syncthreads();
+    floatx4 S[2][4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int row = 32 * (kt >> 1) + 8 * (kt & 1) + 16 * (lr >> 3) + (lr & 7);
+        const u32x4 a = *reinterpret_cast<lds_ptr>(lds0 + row * 128 + ((4 * s + g4) ^ swz(row)) * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) S[i][kt] = mfma16(a, qf[i][s], s == 0 ? zero4 : S[i][kt]);
+      }
+    u32x4 pb[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + 16 * (g4 >> 1) + 4 * (g4 & 1) + r;
+          S[i][kt][r] = kk < lim ? S[i][kt][r] * p.c : -INFINITY;
+          mx = fmaxf(mx, S[i][kt][r]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = fmaxf(m[i], mx);
+      const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
+      const float off = mn == -INFINITY ? 0.f : mn;
+      m[i] = mn;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        lacc[i][r] *= alpha;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) oacc[i][t][r] *= alpha;
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(S[i][kt][r] - off),
+                                    __builtin_amdgcn_exp2f(S[i][kt][r + 1] - off));
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lacc[i] = mfma16(ones, pb[i][s], lacc[i]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int row = 16 * t + lr;
+        const u32x4 a = *reinterpret_cast<lds_ptr>(lds0 + kTile * 2 + row * 128 + ((4 * s + g4) ^ swz(row)) * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) oacc[i][t] = mfma16(a, pb[i][s], oacc[i][t]);
+      }
+    }
+  }
+  store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
+}
+
+// kDense: every key block instead of a list.
+template <bool kDense>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void bsattn_fwd_kernel(const AttnParams p) {
   constexpr int CH = 512 / kThreads;  // 16-byte chunks per thread per tile
-  __shared__ __attribute__((aligned(16))) uint16_t smem[2][2][kTile];  // [buffer][K, Vt]
-  __shared__ float pv_gap[kPv ? 4 : 1];                                 // per-wave gap of the PV post-cut
-  auto lds_u32 = [](const uint16_t *ptr) { return lds_addr32(ptr); };
+  constexpr uint32_t kBufBytes = 2 * kTile * 2;
+  __shared__ __attribute__((aligned(2 * kBufBytes))) uint16_t smem[2][2][kTile];  // [buffer][K, Vt]
+  __shared__ int redo;  // a wave's row sums left the range of offset 0
 
   // Workgroups [0, num_wg2_slots) take the special-token queries (every key
   // block; the slot count is rounded up to a multiple of the 8 XCDs so that
@@ -146,7 +348,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const int64_t b = bh / p.H;
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform
-  const int l = tid & 63, lr = l & 31, hf = l >> 5;
+  const int l = tid & 63, lr = l & 15, g4 = l >> 4;
 
   int n;
   const int32_t *list = nullptr;
@@ -163,19 +365,266 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const uint16_t *qsrc = sp ? p.q2 : p.q;
   const int64_t q_sb = sp ? p.q2_sb : p.q_sb, q_sh = sp ? p.q2_sh : p.q_sh, q_st = sp ? p.q2_st : p.q_st;
   const int64_t nq = sp ? p.nq2 : p.nq;
-  uint16_t *odst = sp ? p.o2 : p.o;
-  const int64_t o_sb = sp ? p.o2_sb : p.o_sb, o_sh = sp ? p.o2_sh : p.o_sh, o_st = sp ? p.o2_st : p.o_st;
-  const int64_t qrow = static_cast<int64_t>(qb) * kBlockQ + w * 32 + lr;
-  const bool qvalid = qrow < nq;
+  const int64_t row0 = static_cast<int64_t>(qb) * kBlockQ + w * 32;
   // a wave whose 32 rows all lie past the queries (the short last block of
   // the special queries) only stages its share of the tiles
-  const bool idle = static_cast<int64_t>(qb) * kBlockQ + w * 32 >= nq;
-  int64_t orow = qvalid ? qrow : 0;
-  if (p.tok_p > 0) {
-    const int64_t per = sp ? p.tok_s : p.tok_p - p.tok_s;  // queries per frame of this kind
-    orow = (orow / per) * p.tok_p + (sp ? 0 : p.tok_s) + orow % per;
+  const bool idle = row0 >= nq;
+  if (tid == 0) redo = 0;
+
+  // Q as the B operand of S^T = K Q^T: lane holds row lr of tile i, d = 32s + 8 g4 .. +7.
+  u32x4 qf[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int64_t qrow = row0 + 16 * i + lr;
+    const uint16_t *qptr = qsrc + b * q_sb + h * q_sh + (qrow < nq ? qrow : 0) * q_st;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      qf[i][s] = qrow < nq ? *reinterpret_cast<const u32x4 *>(qptr + 32 * s + 8 * g4) : u32x4{0, 0, 0, 0};
   }
-  uint16_t *optr = odst + b * o_sb + h * o_sh + orow * o_st;
+  // consume Q here so that the compiler's wait for these loads lands before
+  // the loop instead of inside it
+  asm volatile("" ::"v"(qf[0][0]), "v"(qf[0][1]), "v"(qf[1][0]), "v"(qf[1][1]));
+
+  // Staging: LDS chunk ci = u*256 + tid lands at byte 16*ci (the DMA writes
+  // lane i of a wave at base + 16*i); it holds tile row ci/8, logical chunk
+  // (ci%8) ^ swizzle(row), so each lane fetches that global chunk. Both
+  // swizzles are the same for row 32u + r as for r: a thread's byte offset
+  // inside the block stays, and the row base (32u rows) goes into the scalar
+  // base address.
+  const uint16_t *kbase = p.k + b * p.k_sb + h * p.k_sh;
+  const uint16_t *vbase = p.vt + (bh * p.nkb) * kTile;
+  const int nk32 = static_cast<int>(p.nk);
+  const int nkb32 = static_cast<int>(p.nkb);
+  const int partial = (nk32 % kBlockK) ? nkb32 - 1 : -1;  // the partial last block, if any
+  const int r0 = tid >> 3;
+  const int kc = ((tid & 7) ^ swz_k(r0)) * 8;
+  const uint32_t koff = static_cast<uint32_t>((static_cast<int64_t>(r0) * p.k_st + kc) * 2);
+  const uint32_t voff = static_cast<uint32_t>((r0 * kHeadDim + ((tid & 7) ^ swz(r0)) * 8) * 2);
+  const uint32_t lds0 = lds_addr32(smem[0][0]);
+  // K and Vt of block blk -> LDS buffer buf. Blocks outside [0, nkb) load
+  // block 0 (the second walk masks them); rows of the partial block past the
+  // sequence end read its last row.
+  auto fetch = [&](int blk, int buf) __attribute__((always_inline)) {
+    const int sb = (blk >= 0 && blk < nkb32) ? blk : 0;
+    const uint16_t *kb = kbase + static_cast<int64_t>(sb) * kBlockK * p.k_st;
+    const uint16_t *vb = vbase + static_cast<int64_t>(sb) * kTile;
+    const uint32_t kd = lds0 + w * 64 * 16 + buf * kBufBytes, vd = kd + kTile * 2;
+    if (sb == partial) {
+      const int last_row = nk32 - 1 - partial * kBlockK;
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int r = 32 * u + r0;
+        const int rr = r < last_row ? r : last_row;
+        dma16(kb, static_cast<uint32_t>((static_cast<int64_t>(rr) * p.k_st + kc) * 2), kd + u * kThreads * 16);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < CH; ++u) dma16(kb + 32 * u * p.k_st, koff, kd + u * kThreads * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) dma16(vb + 32 * u * kHeadDim, voff, vd + u * kThreads * 16);
+  };
+  // Keys of block blk that exist: 64, fewer for the partial last block, 0
+  // for blocks outside [0, nkb).
+  auto valid_keys = [&](int blk) __attribute__((always_inline)) {
+    return (blk >= 0 && blk < nkb32) ? (blk == partial ? nk32 - blk * kBlockK : kBlockK) : 0;
+  };
+
+  const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  const float c = p.c;
+  floatx4 oacc[2][4];  // O^T: [q tile][d tile]
+  floatx4 lacc[2];     // row sums of the bf16 probabilities (every register of every lane group alike)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    lacc[i] = zero4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
+  }
+  // operand addresses in the current buffer: row 16 (lr / 8) + lr % 8 of the
+  // K tile and row lr of the Vt tile, chunk 4 s + g4
+  typedef const __attribute__((address_space(3))) u32x4 *lds_ptr;
+  const int krow = 16 * (lr >> 3) + (lr & 7);
+  uint32_t ka_addr[2], va_addr[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    ka_addr[s] = lds0 + krow * 128 + ((4 * s + g4) ^ swz_k(krow)) * 16;
+    va_addr[s] = lds0 + kTile * 2 + lr * 128 + ((4 * s + g4) ^ swz(lr)) * 16;
+  }
+  auto k_op = [&](int kt, int s) {
+    return *reinterpret_cast<lds_ptr>(ka_addr[s] + (32 * (kt >> 1) + 8 * (kt & 1)) * 128);
+  };
+  auto v_op = [&](int t, int s) { return *reinterpret_cast<lds_ptr>(va_addr[s] + 16 * t * 128); };
+  // The A operand of the row sums: ones, zero at keys at or past lim.
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+  u32x4 sum_a[2] = {ones, ones};
+  auto set_ones = [&](int lim) __attribute__((always_inline)) {
+    int lane_key = 16 * (g4 >> 1) + 4 * (g4 & 1);
+    asm volatile("" : "+v"(lane_key));  // keeps the per-key compares out of the loop's registers
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int kk = 32 * s + 8 * (e >> 1) + lane_key + 2 * (e & 1);
+        sum_a[s][e] = kk + 1 < lim ? 0x3f803f80u : (kk < lim ? 0x3f80u : 0u);
+      }
+  };
+  // Probabilities at offset 0 and their products with Vt.
+  auto compute = [&]() __attribute__((always_inline)) {
+    floatx4 S[2][4];
+    u32x4 ka[4][2];  // all K operands of the block, read before the first product
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) ka[kt][s] = k_op(kt, s);
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) S[i][kt] = mfma16(ka[kt][s], qf[i][s], s == 0 ? zero4 : S[i][kt]);
+    u32x4 pb[2][2];  // [q tile][32-key group]
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(S[i][kt][r] * c),
+                                    __builtin_amdgcn_exp2f(S[i][kt][r + 1] * c));
+        }
+    u32x4 va[4][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) va[t][s] = v_op(t, s);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        lacc[i] = mfma16(sum_a[s], pb[i][s], lacc[i]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) oacc[i][t] = mfma16(va[t][s], pb[i][s], oacc[i][t]);
+      }
+    // every K read issued before the first score product, then the products,
+    // the exponentials, the Vt reads and the products with them
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+    __builtin_amdgcn_sched_group_barrier(0x402, 80, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 20, 0);
+  };
+  // A row sum out of range, infinite or NaN (bit patterns, so that NaN
+  // compares as well).
+  auto sums_bad = [&]() __attribute__((always_inline)) {
+    bool x = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x |= __float_as_uint(lacc[i][0]) - kLowBits > kHighBits - kLowBits;
+    return __ballot(x) != 0;
+  };
+
+  // List entry j+1 is loaded during iteration j-1 (index clamped to the list)
+  // so that reading it never waits on memory: the wait at the top of each
+  // iteration already covers it.
+  const __attribute__((address_space(4))) int32_t *clist =
+      (const __attribute__((address_space(4))) int32_t *)(list);
+  bool out_of_list = false;  // a block outside the sequence was listed
+  // The walk: wait for a block's tiles, start the next block's DMA into the
+  // other buffer, compute. kIdle: a wave without rows, which only stages its
+  // share of the tiles and keeps the barriers.
+  auto walk = [&](auto idle_wave) __attribute__((always_inline)) {
+    constexpr bool kIdle = decltype(idle_wave)::value;
+    int blk = dense ? 0 : clist[0];
+    int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
+    fetch(blk, 0);
+    int nw = n;
+#pragma clang loop unroll(disable)
+    for (int j = 0; j < nw; ++j) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (j == kCheckAt && __builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
+      const int lim = valid_keys(blk);
+      if (j + 1 < nw) {
+        if (dense) {
+          blk = j + 1;
+        } else {
+          const int e = e_next;
+          blk = p.delta ? blk + e : e;
+          e_next = clist[j + 2 < n ? j + 2 : n - 1];
+        }
+        fetch(blk, (j & 1) ^ 1);
+      }
+      if constexpr (!kIdle) {
+        if (__builtin_expect(lim < kBlockK, 0)) {
+          set_ones(lim);
+          out_of_list |= lim == 0;
+        }
+        compute();
+        if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
+        if (j == kCheckAt - 1 && sums_bad()) redo = 1;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          ka_addr[s] ^= kBufBytes;
+          va_addr[s] ^= kBufBytes;
+        }
+      }
+    }
+  };
+  if (n > 0) {
+    if (idle) {
+      walk(std::true_type{});
+    } else {
+      walk(std::false_type{});
+      uint32_t top = 0;  // largest magnitude of O, as bits
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const uint32_t o = __float_as_uint(oacc[i][t][r]) & 0x7fffffffu;
+            top = o > top ? o : top;
+          }
+      if (sums_bad() || __ballot(top >= 0x7f800000u) != 0 || out_of_list) redo = 1;
+    }
+  }
+
+  store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
+  // last, so that no result lives across the call: its stores follow these
+  __syncthreads();  // every wave is done with the tiles and with redo
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0))
+    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()), lds0,
+                  kDense, static_cast<int>(wg), n);
+}
+
+// The PV post-cut (qk_int_sv_f16_cuda_sm80.cuh:291-381): 4 waves x 32 query
+// rows on v_mfma_f32_32x32x16_bf16 (a lane owns row lane % 32 and 32 of the
+// 64 keys), with the exponent offset m moved per block where its sums leave
+// the range. Its execution map is kept per 32-row wave.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void bsattn_pv_kernel(const AttnParams p) {
+  constexpr int CH = 512 / kThreads;  // 16-byte chunks per thread per tile
+  __shared__ __attribute__((aligned(16))) uint16_t smem[2][2][kTile];  // [buffer][K, Vt]
+  __shared__ float pv_gap[4];                                           // per-wave gap of the PV post-cut
+  auto lds_u32 = [](const uint16_t *ptr) { return lds_addr32(ptr); };
+
+  const int64_t nqb = p.nqb;
+  const int64_t wg = p.head_major ? static_cast<int64_t>(blockIdx.x) : xcd_remap(blockIdx.x, p.num_wg);
+  const int qb = static_cast<int>(wg % nqb);
+  const int64_t bh = wg / nqb;
+  const int64_t h = bh % p.H;
+  const int64_t b = bh / p.H;
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform
+  const int l = tid & 63, lr = l & 31, hf = l >> 5;
+
+  const int64_t row = bh * p.nqb + qb;
+  const int32_t *list = p.idx + row * p.idx_w;
+  int n = p.cnt[row];
+  n = n < 0 ? 0 : (n > p.idx_w ? static_cast<int>(p.idx_w) : n);
+
+  const int64_t qrow = static_cast<int64_t>(qb) * kBlockQ + w * 32 + lr;
+  const bool qvalid = qrow < p.nq;
+  uint16_t *optr = p.o + b * p.o_sb + h * p.o_sh + (qvalid ? qrow : 0) * p.o_st;
 
   if (n == 0) {
     if (qvalid) {
@@ -188,7 +637,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   // Q as the B operand of S^T = K Q^T: lane holds row lr, d = 16s + 8hf .. +7.
   u32x4 qf[4];
   {
-    const uint16_t *qptr = qsrc + b * q_sb + h * q_sh + (qvalid ? qrow : 0) * q_st;
+    const uint16_t *qptr = p.q + b * p.q_sb + h * p.q_sh + (qvalid ? qrow : 0) * p.q_st;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
       qf[s] = qvalid ? *reinterpret_cast<const u32x4 *>(qptr + 16 * s + 8 * hf) : u32x4{0, 0, 0, 0};
@@ -247,7 +696,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   float m = 0.f;   // exponent offset of this lane's row (log2 units)
   const float c = p.c;
   float run_max = -5000000.0f;  // PV post-cut: running row max (log2 units)
-  const float pv_threshold = kPv ? p.pv_thr[h] : 0.f;
+  const float pv_threshold = p.pv_thr[h];
 
   // P = exp2(c S - m) for k-step s of the PV product (accumulators
   // 8(s%2)..+7 of tile s/2), packed to bf16; returns bs plus the sum of the
@@ -321,8 +770,8 @@ void bsattn_fwd_kernel(const AttnParams p) {
   // iteration already covers it.
   const __attribute__((address_space(4))) int32_t *clist =
       (const __attribute__((address_space(4))) int32_t *)(list);
-  int blk = dense ? 0 : clist[0];
-  int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
+  int blk = clist[0];
+  int32_t e_next = clist[n > 1 ? 1 : 0];
   fetch(blk, 0);
   // One block: wait for its tiles, start the next block's DMA into the other
   // buffer, compute. The loop runs two blocks per trip so that each block's
@@ -331,18 +780,13 @@ void bsattn_fwd_kernel(const AttnParams p) {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     const int cur = blk;
     if (j + 1 < n) {
-      if (dense) {
-        blk = j + 1;
-      } else {
-        const int e = e_next;
-        blk = p.delta ? blk + e : e;
-        e_next = clist[j + 2 < n ? j + 2 : n - 1];
-      }
+      const int e = e_next;
+      blk = p.delta ? blk + e : e;
+      e_next = clist[j + 2 < n ? j + 2 : n - 1];
       fetch(blk, buf ^ 1);
     }
     const uint16_t *ks = smem[buf][0];
     const uint16_t *vs = smem[buf][1];
-    if (!kPv && idle) return;
 
     // S^T tiles: keys 32t + [0,32) x this wave's 32 query rows.
     floatx16 S[2];
@@ -367,51 +811,42 @@ void bsattn_fwd_kernel(const AttnParams p) {
     // workgroup's rows of (block row max - running max) in log2 units; the
     // running max starts at -5e6 and follows every listed block, executed or
     // not; PV runs for the whole workgroup only when gap + threshold > 0.
-    if constexpr (kPv) {
-      if (!dense) {
-        const int lim = valid_keys(cur);
-        float mx = -5000000.0f;
-        if (lim == kBlockK) {  // a whole block (the usual case): no per-key masks
+    const int lim = valid_keys(cur);
+    float mx = -5000000.0f;
+    if (lim == kBlockK) {  // a whole block (the usual case): no per-key masks
 #pragma unroll
-          for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[t][r]);
-        } else {
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[t][r]);
+    } else {
 #pragma unroll
-          for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int kk = 32 * t + 8 * (r >> 2) + 4 * hf + (r & 3);
-              mx = kk < lim ? fmaxf(mx, S[t][r]) : mx;
-            }
+        for (int r = 0; r < 16; ++r) {
+          const int kk = 32 * t + 8 * (r >> 2) + 4 * hf + (r & 3);
+          mx = kk < lim ? fmaxf(mx, S[t][r]) : mx;
         }
-        mx = fmaxf(mx, xor_lane(mx, 32)) * c;
-        float gap = mx - run_max;  // the wave's largest, by VALU cross-lane moves (rows 0-31, both halves)
-#pragma unroll
-        for (int off = 16; off >= 1; off >>= 1) gap = fmaxf(gap, xor_lane(gap, off));
-        run_max = fmaxf(run_max, mx);
-        if (l == 0) pv_gap[w] = gap;
-      }
     }
+    mx = fmaxf(mx, xor_lane(mx, 32)) * c;
+    float gap = mx - run_max;  // the wave's largest, by VALU cross-lane moves (rows 0-31, both halves)
+#pragma unroll
+    for (int off = 16; off >= 1; off >>= 1) gap = fmaxf(gap, xor_lane(gap, off));
+    run_max = fmaxf(run_max, mx);
+    if (l == 0) pv_gap[w] = gap;
 
     // keys past the sequence end (partial or out-of-range blocks) are masked
     // before the exponentials, so such a block stays on the fast path unless
     // its sums leave the range
-    const int lim = valid_keys(cur);
     if (lim < kBlockK) mask_keys(S, lim);
     u32x4 pb[4];
     float bs = exp_block(S, pb);  // changes no state: a skipped block drops it
-    if constexpr (kPv) {
-      if (!dense) {
-        // the workgroup's decision, read after the exponentials so that the
-        // barrier wait overlaps them
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const float g4 = fmaxf(fmaxf(pv_gap[0], pv_gap[1]), fmaxf(pv_gap[2], pv_gap[3]));
-        if (!(g4 + pv_threshold > 0.f)) return;  // skipped: no sum, no PV
-        if (l == 0 && p.pv_map && cur >= 0 && cur < nkb32)
-          p.pv_map[((bh * p.nqb + qb) * 4 + w) * p.pv_w + cur] = 1;
-      }
-    }
+    // the workgroup's decision, read after the exponentials so that the
+    // barrier wait overlaps them
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const float g4 = fmaxf(fmaxf(pv_gap[0], pv_gap[1]), fmaxf(pv_gap[2], pv_gap[3]));
+    if (!(g4 + pv_threshold > 0.f)) return;  // skipped: no sum, no PV
+    if (l == 0 && p.pv_map && cur >= 0 && cur < nkb32)
+      p.pv_map[((bh * p.nqb + qb) * 4 + w) * p.pv_w + cur] = 1;
     if (__ballot(!(bs <= kHigh) || !(ls + bs >= kLow))) bs = slow(S, pb);
     ls += bs;
 
@@ -526,7 +961,9 @@ int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64
   p.tok_p = ot.P;
   p.tok_s = ot.S;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  auto kern = dense ? bsattn_fwd_kernel<true> : (pv_thr ? bsattn_fwd_kernel<false, true> : bsattn_fwd_kernel<false>);
+  auto kern = pv_thr ? bsattn_pv_kernel
+              : dense ? bsattn_fwd_kernel<true>
+                      : bsattn_fwd_kernel<false>;
   hipLaunchKernelGGL(kern, dim3(p.num_wg + p.num_wg2_slots), dim3(kThreads), 0, s, p);
   return check_launch(dense ? "vasc_dense_attn_fwd" : "vasc_block_sparse_attn_fwd");
 }
