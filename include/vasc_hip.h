@@ -480,6 +480,24 @@ int vasc_restore_tokens(const uint16_t *x_patch, int64_t p_sb, int64_t p_sh,
                         int64_t N, int64_t P, int64_t S, int64_t d,
                         uint16_t *out, void *stream);
 
+/* vasc_pack_global with q_patch and q_special written as
+ * bf16(q * q_scale), one rounding after the norm and the rotary embedding
+ * (q_scale > 0; the pooled means stay those of the unscaled bf16 rows).
+ * With q_scale = log2(e) * sm_scale the attention entry points take
+ * sm_scale = ln 2, and the list-driven ones then need no product per score. */
+int vasc_pack_global_scaled(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh,
+                     const uint16_t *k, int64_t k_sb, int64_t k_st, int64_t k_sh,
+                     const uint16_t *v, int64_t v_sb, int64_t v_st, int64_t v_sh,
+                     int64_t B, int64_t H, int64_t N, int64_t P, int64_t S,
+                     int64_t d, const void *q_norm_w, const void *q_norm_b,
+                     float q_eps, int32_t q_norm, const void *k_norm_w,
+                     const void *k_norm_b, float k_eps, int32_t k_norm,
+                     const int32_t *pos, int64_t pos_sb, int64_t pos_st,
+                     const float *rope_cos, const float *rope_sin, int64_t rope_n,
+                     uint16_t *q_patch, uint16_t *q_special, uint16_t *k_out,
+                     uint16_t *vt, uint16_t *pooled_q, uint16_t *pooled_k,
+                     uint16_t *pooled_v, float *innovation, float q_scale, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

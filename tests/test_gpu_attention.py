@@ -221,6 +221,36 @@ def test_range_exit_at_every_point_of_the_walk(nblk, at, reverse, hot):
     _check(ops.dense_attn(qc, kc, vt), ref)
 
 
+@pytest.mark.parametrize("N,P,S,H", [(1, 129, 1, 1), (3, 47, 5, 3), (2, 130, 0, 9)])
+def test_prescaled_queries_match_the_oracle(N, P, S, H):
+    """Queries packed with the softmax scale (one bf16 rounding of q * scale
+    instead of one of q): the layout differs in q only, the pooled means not at
+    all, and the prescaled attention stays within the file's tolerance of the float64 softmax of the unscaled float32 queries."""
+    from vasc_amd import ops
+    T = N * P
+    qkv = _rand((1, T, 3, H, 64), 40).cuda()
+    q, k, v = (qkv[:, :, i] for i in range(3))
+    c = ops.LOG2E / 8.0
+    ref = ops.pack_global(q, k, v, N, P, S)
+    got = ops.pack_global(q, k, v, N, P, S, q_scale=c)
+    for i, (a, b) in enumerate(zip(ref, got)):
+        if a is None:
+            assert b is None
+        elif i < 2:  # q_patch, q_special
+            assert torch.equal(b, (a.float() * torch.tensor(c, dtype=torch.float32, device="cuda")).to(torch.bfloat16))
+        else:
+            assert torch.equal(a, b)
+    qp, qs, ko, vt = got[:4]
+    np_, qb, nkb = N * (P - S), math.ceil(N * (P - S) / 128), math.ceil(T / 64)
+    idx, cnt = _lists(1, H, qb, nkb, 41, density=0.6)
+    rows = OA.block_sparse_attention(ref[0].float().cpu().numpy(), ko.float().cpu().numpy(),
+                                     ops.pack_qkv(q, k, v, N, P, S)[3].float().cpu().numpy(), idx, cnt)
+    out = ops.global_attn_tokens(qp, qs, ko, vt, torch.from_numpy(idx).cuda(), torch.from_numpy(cnt).cuda(), N, P, S,
+                                 scale=ops.LN2)
+    patch = out.view(1, N, P, H, 64)[:, :, S:].reshape(1, np_, H, 64).transpose(1, 2)
+    _check(patch, rows)
+
+
 # ---------------------------------------------------------------- PV post-cut
 def _graded_blocks(nq, nk, levels, seed):
     """Query rows a*e0 (+ small noise) and key block j = levels[j] / c * e0

@@ -48,6 +48,7 @@ struct PackParams {
   int32_t H, N, P, S;           // T = N * P frame-major tokens
   const void *norm_w[2], *norm_b[2];
   float eps[2];
+  float q_scale;                // pack_global_kernel: q is written times this, before its one rounding to bf16
   int32_t norm[2];              // LayerNorm of q (0) and k (1): 0 none, 1 fp32 parameters, 2 bf16 parameters
   const int32_t *pos;           // (row, column) position of token (b, t) at pos + b*pos_sb + t*pos_st
   int64_t pos_sb, pos_st;
@@ -277,7 +278,12 @@ __global__ __launch_bounds__(kThreads) void pack_global_kernel(const PackParams 
         uint16_t *dst = X == 0 ? (patch ? p.q_patch + (bh * np + i) * kHeadDim
                                         : p.q_special + (bh * ns + (i - np)) * kHeadDim)
                                : p.k_out + (bh * T + i) * kHeadDim;
-        *reinterpret_cast<u32x4 *>(dst + sub * 8) = out;
+        u32x4 stored = out;
+        if (X == 0 && p.q_scale != 1.f) {  // the means below stay those of the unscaled rows
+#pragma unroll
+          for (int e = 0; e < 4; ++e) stored[e] = pack_bf16x2(x[2 * e] * p.q_scale, x[2 * e + 1] * p.q_scale);
+        }
+        *reinterpret_cast<u32x4 *>(dst + sub * 8) = stored;
       }
       if (patch) {
 #pragma unroll
@@ -479,7 +485,7 @@ extern "C" int vasc_pack_qkv(const uint16_t *q, int64_t q_sb, int64_t q_st, int6
   return check_launch("vasc_pack_qkv");
 }
 
-extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh, const uint16_t *k,
+static int pack_global_impl(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh, const uint16_t *k,
                                 int64_t k_sb, int64_t k_st, int64_t k_sh, const uint16_t *v, int64_t v_sb,
                                 int64_t v_st, int64_t v_sh, int64_t B, int64_t H, int64_t N, int64_t P, int64_t S,
                                 int64_t d, const void *q_norm_w, const void *q_norm_b, float q_eps, int32_t q_norm,
@@ -487,7 +493,7 @@ extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, i
                                 const int32_t *pos, int64_t pos_sb, int64_t pos_st, const float *rope_cos,
                                 const float *rope_sin, int64_t rope_n, uint16_t *q_patch, uint16_t *q_special,
                                 uint16_t *k_out, uint16_t *vt, uint16_t *pooled_q, uint16_t *pooled_k,
-                                uint16_t *pooled_v, float *innovation, void *stream) {
+                                uint16_t *pooled_v, float *innovation, float q_scale, void *stream) {
   using namespace vasc;
   VASC_SUPPORTED(d == kHeadDim, "head_dim %lld not built (built: 64)", (long long)d);
   VASC_REQUIRE(B > 0 && H > 0 && N > 0 && P > 0 && S >= 0 && S < P, "invalid sizes B=%lld H=%lld N=%lld P=%lld S=%lld",
@@ -513,6 +519,7 @@ extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, i
                  "rotary tables must be 16-byte aligned");
     VASC_REQUIRE(pos_sb >= 0 && pos_st >= 2, "position strides must be pos_sb >= 0, pos_st >= 2");
   }
+  VASC_REQUIRE(q_scale > 0.f && q_scale <= 3.0e38f, "q_scale must be positive and finite");
   PackParams p{};
   p.src[0] = q; p.src[1] = k; p.src[2] = v;
   p.sb[0] = q_sb; p.st[0] = q_st; p.sh[0] = q_sh;
@@ -520,6 +527,7 @@ extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, i
   p.sb[2] = v_sb; p.st[2] = v_st; p.sh[2] = v_sh;
   p.H = static_cast<int32_t>(H); p.N = static_cast<int32_t>(N); p.P = static_cast<int32_t>(P);
   p.S = static_cast<int32_t>(S);
+  p.q_scale = q_scale;
   p.norm_w[0] = q_norm_w; p.norm_b[0] = q_norm_b; p.eps[0] = q_eps; p.norm[0] = q_norm;
   p.norm_w[1] = k_norm_w; p.norm_b[1] = k_norm_b; p.eps[1] = k_eps; p.norm[1] = k_norm;
   p.pos = pos; p.pos_sb = pos_sb; p.pos_st = pos_st;
@@ -530,6 +538,36 @@ extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, i
   hipLaunchKernelGGL(pack_global_kernel, dim3(static_cast<unsigned>(cdiv(N * P, 128) * H), static_cast<unsigned>(B)),
                      dim3(kThreads), 0, reinterpret_cast<hipStream_t>(stream), p);
   return check_launch("vasc_pack_global");
+}
+
+extern "C" int vasc_pack_global(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh, const uint16_t *k,
+                                int64_t k_sb, int64_t k_st, int64_t k_sh, const uint16_t *v, int64_t v_sb,
+                                int64_t v_st, int64_t v_sh, int64_t B, int64_t H, int64_t N, int64_t P, int64_t S,
+                                int64_t d, const void *q_norm_w, const void *q_norm_b, float q_eps, int32_t q_norm,
+                                const void *k_norm_w, const void *k_norm_b, float k_eps, int32_t k_norm,
+                                const int32_t *pos, int64_t pos_sb, int64_t pos_st, const float *rope_cos,
+                                const float *rope_sin, int64_t rope_n, uint16_t *q_patch, uint16_t *q_special,
+                                uint16_t *k_out, uint16_t *vt, uint16_t *pooled_q, uint16_t *pooled_k,
+                                uint16_t *pooled_v, float *innovation, void *stream) {
+  return pack_global_impl(q, q_sb, q_st, q_sh, k, k_sb, k_st, k_sh, v, v_sb, v_st, v_sh, B, H, N, P, S, d, q_norm_w,
+                          q_norm_b, q_eps, q_norm, k_norm_w, k_norm_b, k_eps, k_norm, pos, pos_sb, pos_st, rope_cos,
+                          rope_sin, rope_n, q_patch, q_special, k_out, vt, pooled_q, pooled_k, pooled_v, innovation,
+                          1.f, stream);
+}
+
+extern "C" int vasc_pack_global_scaled(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh, const uint16_t *k,
+                                int64_t k_sb, int64_t k_st, int64_t k_sh, const uint16_t *v, int64_t v_sb,
+                                int64_t v_st, int64_t v_sh, int64_t B, int64_t H, int64_t N, int64_t P, int64_t S,
+                                int64_t d, const void *q_norm_w, const void *q_norm_b, float q_eps, int32_t q_norm,
+                                const void *k_norm_w, const void *k_norm_b, float k_eps, int32_t k_norm,
+                                const int32_t *pos, int64_t pos_sb, int64_t pos_st, const float *rope_cos,
+                                const float *rope_sin, int64_t rope_n, uint16_t *q_patch, uint16_t *q_special,
+                                uint16_t *k_out, uint16_t *vt, uint16_t *pooled_q, uint16_t *pooled_k,
+                                uint16_t *pooled_v, float *innovation, float q_scale, void *stream) {
+  return pack_global_impl(q, q_sb, q_st, q_sh, k, k_sb, k_st, k_sh, v, v_sb, v_st, v_sh, B, H, N, P, S, d, q_norm_w,
+                          q_norm_b, q_eps, q_norm, k_norm_w, k_norm_b, k_eps, k_norm, pos, pos_sb, pos_st, rope_cos,
+                          rope_sin, rope_n, q_patch, q_special, k_out, vt, pooled_q, pooled_k, pooled_v, innovation,
+                          q_scale, stream);
 }
 
 extern "C" int vasc_restore_tokens(const uint16_t *x_patch, int64_t p_sb, int64_t p_sh, int64_t p_st,

@@ -16,6 +16,9 @@ from . import _lib
 BLOCK_Q = 128
 BLOCK_K = 64
 HEAD_DIM = 64
+# the attention kernels' softmax runs in base 2: queries packed with
+# q_scale = LOG2E * scale take scale = LN2 there
+LOG2E, LN2 = 1.4426950408889634, 0.6931471805599453
 
 
 def _stream() -> int:
@@ -562,7 +565,7 @@ def pack_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None, frames: i
 def pack_global(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, frames: int, tokens_per_frame: int,
                 special: int, *, q_norm=None, k_norm=None, pos: torch.Tensor | None = None,
                 rope_tables: tuple[torch.Tensor, torch.Tensor] | None = None, innovation: bool = True,
-                pooled_v: bool = False):
+                pooled_v: bool = False, q_scale: float = 1.0):
     """``pack_qkv`` with V packed straight into attention tiles and the
     block-mean pooling of the patch tokens in the same pass.
 
@@ -571,7 +574,9 @@ def pack_global(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, frames: int, 
     for bit), ``vt`` as ``pack_v`` of the packed V, ``pooled_q`` / ``pooled_k``
     as ``pool_qkv(q_patch, k[:, :, :Np])``, ``innovation`` (or None) the pair
     innovation of the patch values' block means, ``pooled_v`` (or None) those
-    means. Requires at least one patch token per frame.
+    means. With ``q_scale`` the queries are written as ``bf16(q * q_scale)``
+    (``pooled_q`` stays that of the unscaled rows). Requires at least one
+    patch token per frame.
     """
     B, T, H, D = q.shape
     N, P, S = int(frames), int(tokens_per_frame), int(special)
@@ -592,9 +597,9 @@ def pack_global(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, frames: int, 
     pv = torch.empty(B, H, kb, D, **bf) if pooled_v else None
     inn = torch.empty(B, H, (kb + 1) // 2, device=dev, dtype=torch.float32) if innovation else None
     keep, args = _layout_args(B, T, D, q_norm, k_norm, pos, rope_tables)
-    _lib.call("vasc_pack_global", *_btht(q, "q"), *_btht(k, "k"), *_btht(v, "v"), B, H, N, P, S, D, *args,
+    _lib.call("vasc_pack_global_scaled", *_btht(q, "q"), *_btht(k, "k"), *_btht(v, "v"), B, H, N, P, S, D, *args,
               qp.data_ptr(), qs.data_ptr(), ko.data_ptr(), vt.data_ptr(), pq.data_ptr(), pk.data_ptr(), _ptr(pv),
-              _ptr(inn), _stream())
+              _ptr(inn), float(q_scale), _stream())
     del keep
     return qp, (qs if S else None), ko, vt, pq, pk, inn, pv
 

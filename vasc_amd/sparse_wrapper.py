@@ -571,7 +571,7 @@ def sparse_global_attention(q_patch: torch.Tensor, q_special: torch.Tensor | Non
                             num_patch_tokens: int | None = None, want_sparsity: bool = True,
                             _innovation: torch.Tensor | None = None, token_layout: tuple | None = None,
                             _vt: torch.Tensor | None = None, _priority: torch.Tensor | None = None,
-                            **research):
+                            _scale: float | None = None, **research):
     """``block_sparse_attn_cuda`` for a whole global layer: the selection of
     the patch queries as there, and the special-token queries (which the
     reference runs through a dense SDPA, ATT:8464-8484) over every key in
@@ -583,7 +583,9 @@ def sparse_global_attention(q_patch: torch.Tensor, q_special: torch.Tensor | Non
     frame-major ``[B, N*P, H*D]`` output (restore included) and the second
     None. ``_vt``: the values already packed as ``ops.pack_v(value)`` (then
     ``value`` may be None); ``_priority``: ``pooled_score`` cleaned as the
-    ledger stores it (``ops.pooled_softmax(..., priority=True)``)."""
+    ledger stores it (``ops.pooled_softmax(..., priority=True)``);
+    ``_scale``: the softmax scale where it is not ``D ** -0.5`` (``ops.LN2``
+    for queries packed with theirs)."""
     _require_gpu(q_patch, "query")
     if value is None and _vt is None:
         raise ValueError("sparse_global_attention requires the values (or their packed tiles)")
@@ -594,14 +596,15 @@ def sparse_global_attention(q_patch: torch.Tensor, q_special: torch.Tensor | Non
     thr = _pv_threshold(key, layer_idx)
     if thr is None:
         if token_layout is not None:
-            out = ops.global_attn_tokens(q_patch, q_special, key, vt, sel["index"], sel["count"], *token_layout)
+            out = ops.global_attn_tokens(q_patch, q_special, key, vt, sel["index"], sel["count"], *token_layout,
+                                         scale=_scale)
             _record_pv_execution(routing_state)
             return out, None, (_sparsity(sel, total_kblk) if want_sparsity else None)
-        o_patch, o_special = ops.global_attn(q_patch, q_special, key, vt, sel["index"], sel["count"])
+        o_patch, o_special = ops.global_attn(q_patch, q_special, key, vt, sel["index"], sel["count"], scale=_scale)
         _record_pv_execution(routing_state)
     else:  # the post-cut applies to the patch queries; the special queries stay dense
-        o_patch, pv_map = ops.block_sparse_attn_pv(q_patch, key, vt, sel["index"], sel["count"], thr)
-        o_special = None if q_special is None else ops.dense_attn(q_special, key, vt)
+        o_patch, pv_map = ops.block_sparse_attn_pv(q_patch, key, vt, sel["index"], sel["count"], thr, scale=_scale)
+        o_special = None if q_special is None else ops.dense_attn(q_special, key, vt, scale=_scale)
         _record_pv_execution(routing_state, pv_map, pooled_score.shape[-1])
     if token_layout is not None:
         return ops.restore_tokens(o_patch, o_special, *token_layout), None, \
