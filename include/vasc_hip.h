@@ -480,6 +480,32 @@ int vasc_restore_tokens(const uint16_t *x_patch, int64_t p_sb, int64_t p_sh,
                         int64_t N, int64_t P, int64_t S, int64_t d,
                         uint16_t *out, void *stream);
 
+/* Operator inputs in IEEE half (the reference's dtype), rounded to bf16 as they
+ * are read: vasc_pool_qkv with every given tensor in half; V packed as
+ * vasc_pack_v and, with k, K as contiguous bf16 [B,H,nk,d] in the same pass;
+ * vasc_block_sparse_attn_fwd with q and o in half (k bf16; o is the bf16 result
+ * in half). */
+int vasc_pool_qkv_f16(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                  const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                  const uint16_t *v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                  int64_t B, int64_t H, int64_t nq, int64_t nk, int64_t d,
+                  int64_t block_q, int64_t block_k,
+                  uint16_t *pooled_q, uint16_t *pooled_k, uint16_t *pooled_v,
+                  float *innovation, void *stream);
+int vasc_pack_kv_f16(const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t *v,
+                     int64_t v_sb, int64_t v_sh, int64_t v_st, int64_t B, int64_t H, int64_t nk, int64_t d,
+                     uint16_t *k_out, uint16_t *vt, void *stream);
+int vasc_block_sparse_attn_f16_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh,
+                               int64_t q_st, const uint16_t *k, int64_t k_sb,
+                               int64_t k_sh, int64_t k_st, const uint16_t *vt,
+                               uint16_t *o, int64_t o_sb, int64_t o_sh,
+                               int64_t o_st, int64_t B, int64_t H, int64_t nq,
+                               int64_t nk, int64_t d,
+                               const int32_t *block_index, int64_t index_width,
+                               const int32_t *block_count,
+                               int32_t index_is_delta, float sm_scale,
+                               void *stream);
+
 /* vasc_pack_global with q_patch and q_special written as
  * bf16(q * q_scale), one rounding after the norm and the rotary embedding
  * (q_scale > 0; the pooled means stay those of the unscaled bf16 rows).

@@ -284,3 +284,36 @@ def test_pv_post_cut_matches_oracle(nq, nk, thr):
     assert np.array_equal(pv_map.cpu().numpy(), ref_map)
     ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), ex_idx, ex_cnt)
     _check(o, ref)
+
+
+# ------------------------------------------------------------- float16 inputs
+@pytest.mark.parametrize("nq,nk,strided", [(1, 1, False), (127, 63, True), (128, 64, False), (129, 65, True),
+                                           (333, 700, True)])
+def test_half_inputs_equal_their_bf16_casts(nq, nk, strided):
+    """float16 q, k, v read by the kernels give, bit for bit, what their bf16
+    casts give: the pooled means and the innovation, K and the V tiles, the
+    attention (its bf16 result as float16). Values over the whole half range,
+    halves that round up to the next bf16, subnormals and infinities among K
+    and V's casts."""
+    from vasc_amd import ops
+    B, H, D = 1, 3, 64
+    def half(n, seed):
+        t = _rand((B, n, H, D), seed).to(torch.float16).cuda()
+        t[:, :, 0, 1::7] = 1.00390625  # between two bf16 values: ties to even
+        return t.transpose(1, 2) if strided else t.transpose(1, 2).contiguous()
+    q, k, v = half(nq, 50), half(nk, 51), half(nk, 52)
+    qc, kc, vc = (t.to(torch.bfloat16) for t in (q, k, v))
+    edge = torch.tensor([65504.0, -65504.0, 6.1e-5, 5.96e-8, -5.96e-8, 0.0, -0.0, float("inf")], dtype=torch.float16)
+    w = k.clone()
+    w[..., :8] = edge.cuda()
+    wk, wt = ops.pack_kv_half(w, w)
+    assert torch.equal(wk.view(torch.int16), w.to(torch.bfloat16).contiguous().view(torch.int16))
+    assert torch.equal(wt.view(torch.int16), ops.pack_v(w.to(torch.bfloat16)).view(torch.int16))
+    for a, b in zip(ops.pool_qkv(q, k, v), ops.pool_qkv(qc, kc, vc)):
+        assert torch.equal(a, b)
+    kb, vt = ops.pack_kv_half(k, v)
+    assert torch.equal(kb, kc) and torch.equal(vt, ops.pack_v(vc)) and torch.equal(vt, ops.pack_v(v))
+    idx, cnt = (torch.from_numpy(t).cuda() for t in _lists(B, H, math.ceil(nq / 128), math.ceil(nk / 64), 53, 0.6))
+    ref = ops.block_sparse_attn(qc, kc, vt, idx, cnt)
+    assert torch.equal(ops.block_sparse_attn(q, kb, vt, idx, cnt), ref)
+    assert torch.equal(ops.block_sparse_attn(q, kb, vt, idx, cnt, half_out=True), ref.to(torch.float16))

@@ -33,6 +33,8 @@ SIGNATURES: dict[str, tuple] = {
                                   P, P, P]),
     "vasc_pool_qkv": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64,
                                 I64, I64, I64, I64, I64, I64, I64, P, P, P, P, P]),
+    "vasc_pool_qkv_f16": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64,
+                                I64, I64, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "vasc_pooled_softmax": (c_int32, [P, P, I64, I64, I64, I64, I64, c_float, I32, P, P, P, P]),
     "vasc_pooled_softmax_workspace_size": (I64, [I64, I64, I64, I64]),
     "vasc_pair_innovation": (c_int32, [P, I64, I64, I64, I64, P, P]),
@@ -47,7 +49,10 @@ SIGNATURES: dict[str, tuple] = {
     "vasc_priority_order": (c_int32, [P, P, P, I64, I32, I64, I64, I64, P, P]),
     "vasc_packed_v_elems": (c_int64, [I64, I64, I64, I64]),
     "vasc_pack_v": (c_int32, [P, I64, I64, I64, I64, I64, I64, I64, P, P]),
+    "vasc_pack_kv_f16": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, I64, I64, I64, I64, P, P, P]),
     "vasc_block_sparse_attn_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, P, I64, I64, I64,
+                                             I64, I64, I64, I64, I64, P, I64, P, I32, c_float, P]),
+    "vasc_block_sparse_attn_f16_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, P, I64, I64, I64,
                                              I64, I64, I64, I64, I64, P, I64, P, I32, c_float, P]),
     "vasc_block_sparse_attn_pv_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, P, I64, I64, I64,
                                                 I64, I64, I64, I64, I64, P, I64, P, I32, c_float, P, P, P]),

@@ -93,6 +93,7 @@ struct AttnParams {
   // token-major output (tok_p > 0): query rows land on the frame-major token
   // rows of o (frames of tok_p tokens, tok_s special ones first)
   int64_t tok_p, tok_s;
+  int32_t half_io;  // q and o are IEEE halves: q rounded to bf16 as it is read, o the bf16 result widened
   // 1: workgroups in hardware order, head-major (sequences whose K and V of
   // eight heads, one per XCD, would overflow the Infinity Cache); 0: each
   // XCD walks a contiguous range of query blocks
@@ -175,6 +176,7 @@ __device__ __forceinline__ void store_rows(const Params &p, bool sp, int64_t b, 
       uint2 v;
       v.x = pack_bf16x2(oacc[i][t][0] * inv, oacc[i][t][1] * inv);
       v.y = pack_bf16x2(oacc[i][t][2] * inv, oacc[i][t][3] * inv);
+      if (p.half_io) v = uint2{bf16x2_to_half2(v.x), bf16x2_to_half2(v.y)};
       *reinterpret_cast<uint2 *>(optr + 16 * t + 4 * g4) = v;
     }
   }
@@ -216,6 +218,9 @@ __device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_a
     for (int s = 0; s < 2; ++s)
       qf[i][s] = qrow < nq ? *reinterpret_cast<const u32x4 *>(qsrc + qrow * q_st + 32 * s + 8 * g4) : u32x4{0, 0, 0, 0};
   }
+  if (p.half_io)
+    for (int i = 0; i < 2; ++i)
+      for (int s = 0; s < 2; ++s) qf[i][s] = half8_to_bf16(qf[i][s]);
   const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
   const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
   floatx4 oacc[2][4], lacc[2];
@@ -384,6 +389,12 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
       qf[i][s] = qrow < nq ? *reinterpret_cast<const u32x4 *>(qptr + 32 * s + 8 * g4) : u32x4{0, 0, 0, 0};
+  }
+  if (p.half_io) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) qf[i][s] = half8_to_bf16(qf[i][s]);
   }
   // consume Q here so that the compiler's wait for these loads lands before
   // the loop instead of inside it
@@ -920,7 +931,7 @@ int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64
                 int64_t nq, int64_t nk, int64_t d, const int32_t *idx, int64_t idx_w,
                 const int32_t *cnt, int32_t delta, float sm_scale, void *stream,
                 const SpecialQueries &sq = SpecialQueries(), const float *pv_thr = nullptr,
-                int32_t *pv_map = nullptr, const OutTokens &ot = OutTokens()) {
+                int32_t *pv_map = nullptr, const OutTokens &ot = OutTokens(), bool half_io = false) {
   VASC_SUPPORTED(d == kHeadDim, "head_dim %lld not built (built: 64)", (long long)d);
   VASC_REQUIRE(B > 0 && H > 0 && nq > 0 && nk > 0, "sizes must be positive");
   int rc;
@@ -964,6 +975,7 @@ int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64
   p.pv_w = p.nkb;
   p.tok_p = ot.P;
   p.tok_s = ot.S;
+  p.half_io = half_io ? 1 : 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   auto kern = pv_thr ? bsattn_pv_kernel
               : dense      ? bsattn_fwd_kernel<true, false>
@@ -986,6 +998,18 @@ extern "C" int vasc_block_sparse_attn_fwd(const uint16_t *q, int64_t q_sb, int64
   return vasc::launch_attn(false, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, vt, o, o_sb, o_sh, o_st, B, H,
                            nq, nk, d, block_index, index_width, block_count, index_is_delta, sm_scale,
                            stream);
+}
+
+extern "C" int vasc_block_sparse_attn_f16_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                                          const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                          const uint16_t *vt, uint16_t *o, int64_t o_sb, int64_t o_sh,
+                                          int64_t o_st, int64_t B, int64_t H, int64_t nq, int64_t nk,
+                                          int64_t d, const int32_t *block_index, int64_t index_width,
+                                          const int32_t *block_count, int32_t index_is_delta,
+                                          float sm_scale, void *stream) {
+  return vasc::launch_attn(false, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, vt, o, o_sb, o_sh, o_st, B, H,
+                           nq, nk, d, block_index, index_width, block_count, index_is_delta, sm_scale,
+                           stream, vasc::SpecialQueries(), nullptr, nullptr, vasc::OutTokens(), true);
 }
 
 extern "C" int vasc_block_sparse_attn_pv_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st,

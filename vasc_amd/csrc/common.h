@@ -70,6 +70,28 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
+// Eight IEEE halves -> eight bf16 (each rounded to nearest even, as a cast of
+// the tensor rounds; NaN -> canonical quiet NaN).
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4 half8_to_bf16(const u32x4 &h) {
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t pair = h[e];  // a copy: a bit cast of the element itself reads element 0
+    const halfx2 v = __builtin_bit_cast(halfx2, pair);
+    o[e] = f32_to_bf16(static_cast<float>(v[0])) |
+           static_cast<uint32_t>(f32_to_bf16(static_cast<float>(v[1]))) << 16;
+  }
+  return o;
+}
+
+// A packed bf16 pair -> the same values as a packed half pair.
+__device__ __forceinline__ uint32_t bf16x2_to_half2(uint32_t pair) {
+  const halfx2 v = {static_cast<_Float16>(__uint_as_float(pair << 16)),
+                    static_cast<_Float16>(__uint_as_float(pair & 0xffff0000u))};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
 // Cross-lane moves inside groups of 8 lanes by DPP: xor 1 and xor 2 are
 // quad permutations, and the half-row mirror (lane i <-> 7 - i) reaches the
 // other quad of the group.

@@ -42,7 +42,9 @@ struct PoolParams {
 // kMax: block max of Q and K instead of the mean (predict_attention with
 // pool_mode="max", F.max_pool1d with ceil_mode: a tail block takes the max of
 // its real tokens). The max of bf16 values is exact; V is not pooled here.
-template <bool kMax>
+// kHalf: the inputs are IEEE halves, each rounded to bf16 as it is read (the
+// rounding a cast of the whole tensor would make in a pass of its own).
+template <bool kMax, bool kHalf>
 __global__ __launch_bounds__(256) void pool_qkv_kernel(const PoolParams p) {
   __shared__ float red[3][2][4][kHeadDim];
   __shared__ float pv[2][kHeadDim];
@@ -79,6 +81,7 @@ __global__ __launch_bounds__(256) void pool_qkv_kernel(const PoolParams p) {
       for (int i = 0; i < 8; ++i) acc[half][i] = kMax ? -INFINITY : 0.f;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
+      if (kHalf) raw[X][u] = half8_to_bf16(raw[X][u]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float lo = __uint_as_float(raw[X][u][i] << 16), hi = __uint_as_float(raw[X][u][i] & 0xffff0000u);
@@ -576,7 +579,7 @@ int pool_impl(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const
                              int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t *v, int64_t v_sb,
                              int64_t v_sh, int64_t v_st, int64_t B, int64_t H, int64_t nq, int64_t nk, int64_t d,
                              int64_t block_q, int64_t block_k, uint16_t *pooled_q, uint16_t *pooled_k,
-                             uint16_t *pooled_v, float *innovation, void *stream, bool pool_max) {
+                             uint16_t *pooled_v, float *innovation, void *stream, bool pool_max, bool half) {
   VASC_SUPPORTED(d == 64 && block_q == 128 && block_k == 64,
                  "pooling variant d=%lld block_q=%lld block_k=%lld not built (built: 64/128/64)", (long long)d,
                  (long long)block_q, (long long)block_k);
@@ -615,12 +618,10 @@ int pool_impl(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const
   p.npairs = cdiv(p.nblk[2], 2);
   const int64_t chunks = cdiv(q ? nq : 0, 128) > cdiv(nk, 128) ? cdiv(nq, 128) : cdiv(nk, 128);
   VASC_REQUIRE(chunks < (int64_t(1) << 31) && B * H < 65536, "grid too large");
-  if (pool_max)
-    hipLaunchKernelGGL(pool_qkv_kernel<true>, dim3(chunks, B * H), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                       p);
-  else
-    hipLaunchKernelGGL(pool_qkv_kernel<false>, dim3(chunks, B * H), dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), p);
+  auto kern = pool_max ? pool_qkv_kernel<true, false>
+              : half   ? pool_qkv_kernel<false, true>
+                       : pool_qkv_kernel<false, false>;
+  hipLaunchKernelGGL(kern, dim3(chunks, B * H), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
   return check_launch(pool_max ? "vasc_pool_qk_max" : "vasc_pool_qkv");
 }
 }  // namespace
@@ -632,7 +633,16 @@ extern "C" int vasc_pool_qkv(const uint16_t *q, int64_t q_sb, int64_t q_sh, int6
                              int64_t block_q, int64_t block_k, uint16_t *pooled_q, uint16_t *pooled_k,
                              uint16_t *pooled_v, float *innovation, void *stream) {
   return vasc::pool_impl(q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st, B, H, nq, nk, d, block_q,
-                         block_k, pooled_q, pooled_k, pooled_v, innovation, stream, false);
+                         block_k, pooled_q, pooled_k, pooled_v, innovation, stream, false, false);
+}
+
+extern "C" int vasc_pool_qkv_f16(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const uint16_t *k,
+                             int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t *v, int64_t v_sb,
+                             int64_t v_sh, int64_t v_st, int64_t B, int64_t H, int64_t nq, int64_t nk, int64_t d,
+                             int64_t block_q, int64_t block_k, uint16_t *pooled_q, uint16_t *pooled_k,
+                             uint16_t *pooled_v, float *innovation, void *stream) {
+  return vasc::pool_impl(q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st, B, H, nq, nk, d, block_q,
+                         block_k, pooled_q, pooled_k, pooled_v, innovation, stream, false, true);
 }
 
 extern "C" int vasc_pool_qk_max(const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const uint16_t *k,
@@ -640,7 +650,7 @@ extern "C" int vasc_pool_qk_max(const uint16_t *q, int64_t q_sb, int64_t q_sh, i
                                 int64_t nk, int64_t d, int64_t block_q, int64_t block_k, uint16_t *pooled_q,
                                 uint16_t *pooled_k, void *stream) {
   return vasc::pool_impl(q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, nullptr, 0, 0, 8, B, H, nq, nk, d, block_q,
-                         block_k, pooled_q, pooled_k, nullptr, nullptr, stream, true);
+                         block_k, pooled_q, pooled_k, nullptr, nullptr, stream, true, false);
 }
 
 extern "C" int vasc_pair_innovation(const float *pooled_v, int64_t B, int64_t H, int64_t kb, int64_t d,

@@ -30,13 +30,13 @@ def _dev(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be a GPU tensor (the HIP path has no CPU fallback)")
 
 
-def _bhtd(t: torch.Tensor, name: str) -> torch.Tensor:
-    """bf16 [B,H,T,D] with unit stride on D and 16-byte aligned rows."""
+def _bhtd(t: torch.Tensor, name: str, dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
+    """``dtype`` [B,H,T,D] with unit stride on D and 16-byte aligned rows."""
     _dev(t, name)
     if t.dim() != 4:
         raise ValueError(f"{name} must be [B,H,T,D], got {tuple(t.shape)}")
-    if t.dtype != torch.bfloat16:
-        t = t.to(torch.bfloat16)
+    if t.dtype != dtype:
+        t = t.to(dtype)
     if t.stride(-1) != 1 or any(s % 8 for s in t.stride()[:3]) or t.data_ptr() % 16:
         t = t.contiguous()
     return t
@@ -67,10 +67,14 @@ def pool_qkv(q=None, k=None, v=None, *, innovation: bool = True):
     Returns ``(pooled_q, pooled_k, pooled_v, innovation)`` with ``None`` for
     skipped inputs.
     """
-    ref = next(t for t in (q, k, v) if t is not None)
-    q = None if q is None else _bhtd(q, "q")
-    k = None if k is None else _bhtd(k, "k")
-    v = None if v is None else _bhtd(v, "v")
+    given = [t for t in (q, k, v) if t is not None]
+    ref = given[0]
+    # float16 tensors are rounded to bf16 as the kernel reads them
+    half = all(isinstance(t, torch.Tensor) and t.dtype == torch.float16 for t in given)
+    dtype = torch.float16 if half else torch.bfloat16
+    q = None if q is None else _bhtd(q, "q", dtype)
+    k = None if k is None else _bhtd(k, "k", dtype)
+    v = None if v is None else _bhtd(v, "v", dtype)
     B, H, _, D = ref.shape
     nq = q.shape[2] if q is not None else 0
     nk = (k if k is not None else v).shape[2] if (k is not None or v is not None) else 0
@@ -82,7 +86,7 @@ def pool_qkv(q=None, k=None, v=None, *, innovation: bool = True):
     if v is not None and innovation:
         inn = torch.empty(B, H, math.ceil(math.ceil(nk / BLOCK_K) / 2), device=dev, dtype=torch.float32)
     st = lambda t: (0, 0, 0) if t is None else tuple(t.stride()[:3])  # noqa: E731
-    _lib.call("vasc_pool_qkv", _ptr(q), *st(q), _ptr(k), *st(k), _ptr(v), *st(v),
+    _lib.call("vasc_pool_qkv_f16" if half else "vasc_pool_qkv", _ptr(q), *st(q), _ptr(k), *st(k), _ptr(v), *st(v),
               B, H, nq, nk, D, BLOCK_Q, BLOCK_K, _ptr(pq), _ptr(pk), _ptr(pv), _ptr(inn), _stream())
     return pq, pk, pv, inn
 
@@ -272,6 +276,8 @@ def settle_terminal(debt, pending_arrival, service) -> torch.Tensor:
 # ----------------------------------------------------------------- kernel 3
 def pack_v(v: torch.Tensor) -> torch.Tensor:
     """Packed, transposed, key-permuted V tiles ``[B,H,ceil(T/64),64,64]`` (bf16)."""
+    if isinstance(v, torch.Tensor) and v.dtype == torch.float16:
+        return pack_kv_half(None, v)[1]
     v = _bhtd(v, "v")
     B, H, T, D = v.shape
     nkb = math.ceil(T / BLOCK_K)
@@ -280,12 +286,31 @@ def pack_v(v: torch.Tensor) -> torch.Tensor:
     return vt
 
 
+def pack_kv_half(k: torch.Tensor | None, v: torch.Tensor):
+    """``(k in bf16 or None, pack_v(v))`` of float16 K and V in one pass."""
+    v = _bhtd(v, "v", torch.float16)
+    B, H, T, D = v.shape
+    vt = torch.empty(B, H, math.ceil(T / BLOCK_K), D, BLOCK_K, device=v.device, dtype=torch.bfloat16)
+    ko, ks = None, (None, 0, 0, 8)
+    if k is not None:
+        k = _bhtd(k, "k", torch.float16)
+        if k.shape != v.shape:
+            raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} differ")
+        ko = torch.empty(B, H, T, D, device=v.device, dtype=torch.bfloat16)
+        ks = (k.data_ptr(), *k.stride()[:3])
+    _lib.call("vasc_pack_kv_f16", *ks, v.data_ptr(), *v.stride()[:3], B, H, T, D, _ptr(ko), vt.data_ptr(), _stream())
+    return ko, vt
+
+
 # ----------------------------------------------------------------- kernel 4
 def block_sparse_attn(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, index: torch.Tensor,
                       count: torch.Tensor, *, scale: float | None = None, delta: bool = False,
-                      out: torch.Tensor | None = None) -> torch.Tensor:
-    """Block-sparse attention over listed 64-key blocks; bf16 output ``[B,H,Nq,D]``."""
-    q = _bhtd(q, "q")
+                      out: torch.Tensor | None = None, half_out: bool = False) -> torch.Tensor:
+    """Block-sparse attention over listed 64-key blocks; bf16 output ``[B,H,Nq,D]``.
+    ``half_out``: the bf16 result as float16, for float16 q (which the kernel
+    then reads as it is)."""
+    half = half_out and q.dtype == torch.float16 and out is None
+    q = _bhtd(q, "q", torch.float16 if half else torch.bfloat16)
     k = _bhtd(k, "k")
     _dev(vt, "vt")
     B, H, nq, D = q.shape
@@ -297,11 +322,13 @@ def block_sparse_attn(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, index:
     count = count.to(torch.int32).contiguous()
     if index.shape[:3] != (B, H, qb) or count.shape != (B, H, qb):
         raise ValueError(f"index/count must be [B,H,{qb},W]/[B,H,{qb}]")
-    o = out if out is not None else torch.empty(B, H, nq, D, device=q.device, dtype=torch.bfloat16)
+    o = out if out is not None else torch.empty(B, H, nq, D, device=q.device, dtype=q.dtype)
     scale = D ** -0.5 if scale is None else scale
-    _lib.call("vasc_block_sparse_attn_fwd", q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3],
+    _lib.call("vasc_block_sparse_attn_f16_fwd" if half else "vasc_block_sparse_attn_fwd", q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3],
               vt.data_ptr(), o.data_ptr(), *o.stride()[:3], B, H, nq, nk, D, index.data_ptr(),
               index.shape[-1], count.data_ptr(), int(bool(delta)), float(scale), _stream())
+    if half_out and not half:
+        o = o.to(torch.float16)
     return o
 
 

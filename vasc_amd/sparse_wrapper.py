@@ -549,10 +549,13 @@ def block_sparse_attn_cuda(query: torch.Tensor, key: torch.Tensor, value: torch.
     _require_gpu(query, "query")
     sel, total_kblk = _select_for_layer(key, value, pooled_score, topk, sparse_ratio, cdf_threshold, layer_idx,
                                         routing_stats_store, routing_state, num_patch_tokens, research)
-    vt = ops.pack_v(value)
     thr = _pv_threshold(key, layer_idx)
+    if key.dtype == value.dtype == torch.float16 and key.shape == value.shape:
+        key, vt = ops.pack_kv_half(key, value)  # one pass over both
+    else:
+        vt = ops.pack_v(value)
     if thr is None:
-        o = ops.block_sparse_attn(query, key, vt, sel["index"], sel["count"])
+        o = ops.block_sparse_attn(query, key, vt, sel["index"], sel["count"], half_out=query.dtype == torch.float16)
         _record_pv_execution(routing_state)
     else:
         o, pv_map = ops.block_sparse_attn_pv(query, key, vt, sel["index"], sel["count"], thr)
