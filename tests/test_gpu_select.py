@@ -330,6 +330,26 @@ def test_cdf_counts_row_kinds_bit_exact(K):
             assert np.array_equal(base.cpu().numpy(), n + (fl & ~last_in & (n < K))), (thr, min_count, fl)
 
 
+@pytest.mark.parametrize("K", [1, 2, 63, 64, 65, 256, 257, 576, 577, 1024, 1087, 1088, 1089, 2047, 2048, 2049])
+def test_cdf_counts_at_the_edges_of_the_row_kernels(K):
+    """Rows at the register and stretch boundaries of the counting kernels,
+    every row kind, counts bit-exact with the oracle; plus rows of one repeated
+    value and of dyadic values, whose every addition is a rounding tie or exact."""
+    rng = np.random.default_rng(900 + K)
+    score = _cdf_rows(rng, K, 14)
+    score = np.concatenate([score, np.full((1, K), 1.0 / K, np.float32),
+                            (rng.integers(1, 5, (1, K)) * np.float32(2.0 ** -13) + np.float32(2.0 ** -25))])
+    score = np.ascontiguousarray(score.astype(np.float32).reshape(1, 1, -1, K))
+    from vasc_amd import ops
+    s = torch.from_numpy(score).cuda()
+    for thr in (0.25, 0.9, 1.0):
+        cnt, base = ops.cdf_counts(s, thr, min_count=0, force_last=True, want_base=True)
+        n = OS.cdf_counts(score, thr, 0)
+        assert np.array_equal(cnt.cpu().numpy(), n), (K, thr)
+        last_in = OS.select_top(score, n)[..., K - 1]
+        assert np.array_equal(base.cpu().numpy(), n + (~last_in & (n < K))), (K, thr)
+
+
 def test_cdf_counts_c5_rows_bit_exact():
     """C5's 4096-block rows (pooled softmax of near-uniform logits), 64 rows
     at the two benchmark thresholds."""

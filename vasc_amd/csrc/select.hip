@@ -188,7 +188,239 @@ __global__ __launch_bounds__(256) void cdf_count_kernel(const float *score, int6
   }
 }
 
-// The same count with the row sorted by rocPRIM's LDS block radix sort (256
+// The same count for rows of up to 2048 key blocks, one wave per row (EPT keys
+// a lane). Bound by instruction issue: about 3500 VALU and 1600 SALU
+// instructions a row of 1036 blocks, half of them in the sort.
+//   sort  1024 buckets of equal key width over the positive keys' range
+//         (counting pass, scan, scatter), then each key's place among its
+//         bucket's few keys. The last bucket takes the keys <= +0, which need no
+//         order while they are all zeros. A row with a bucket above kBigBucket
+//         keys (infinities beside probabilities, planted ties) goes through a
+//         bitonic network instead.
+//   walk  the float32 running sum S of the sorted values is sequential, but
+//         while it stays in one binade [2^e, 2^(e+1)) every addend x rounds to a
+//         multiple of 2^(e-23) by itself, unless x lies half way between two (a
+//         tie, which the parity of S decides). So lane l takes the l-th stretch of
+//         kC sorted values, sums their rounded multiples, and a wave scan gives S
+//         at the end of every stretch, exactly, as long as S stays below 2^(e+1).
+//         The first stretch that holds a tie or a value that is not finite and
+//         non-negative, or ends past the binade or past T, is added one by one;
+//         the scan then resumes behind it.
+// Against the radix kernel below: 1036 blocks x 8288 rows 164 -> 97 us, 1024
+// blocks x 8192 rows 102-135 -> 74-94 us; at 4096 blocks, where a row needs
+// four waves, this scheme took 1.8-2.3 ms against 1.2-1.6, so the longer rows
+// stay there.
+constexpr int kCdfBins = 1024, kBigBucket = 48;
+// Exponent distance of S from a stretch's largest value below which the
+// stretch is added one by one at once: the chance of a tie in it is about
+// kC 2^-distance.
+constexpr int kCdfTieGap = 6;
+template <int EPT>
+__global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, int64_t H, int64_t Q, int K,
+                                                              const float *thr, int32_t min_count, int32_t force_last,
+                                                              int32_t *count_out, int32_t *base_out) {
+  constexpr int kRow = 64 * EPT;
+  constexpr int kC = EPT | 1;          // values per stretch (odd: the lanes' reads spread over the banks)
+  constexpr int kOwn = kCdfBins / 64;
+  // the row, grouped and then sorted in place, and the bins; the bitonic
+  // network takes both: the power of two above K fits (K <= kRow)
+  __shared__ __attribute__((aligned(16))) uint32_t buf[kRow + kCdfBins + 4];
+  static_assert(kRow + kCdfBins >= 2048 || kRow <= 1024, "room for the network");
+  uint32_t *bins = buf + kRow;
+  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x;
+  const float *srow = score + row * K;
+  const uint32_t last = order_key(srow[K - 1]);
+  constexpr uint32_t kZero = 0x80000000u;  // the key of 0
+  uint32_t key[EPT];
+  uint32_t kmin = 0xffffffffu, kpos = 0xffffffffu, kmax = 0u;
+  int beat = 0;
+#pragma unroll
+  for (int m = 0; m < EPT; ++m) {
+    const int k = lane + 64 * m;
+    key[m] = k < K ? order_key(srow[k]) : 0u;  // no value has the key 0
+    if (k < K) {
+      kmin = min(kmin, key[m]);
+      kmax = max(kmax, key[m]);
+      if (key[m] > kZero) kpos = min(kpos, key[m]);
+    }
+    beat += k < K - 1 && key[m] >= last;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    kmin = min(kmin, static_cast<uint32_t>(__shfl_xor(static_cast<int>(kmin), o)));
+    kpos = min(kpos, static_cast<uint32_t>(__shfl_xor(static_cast<int>(kpos), o)));
+    kmax = max(kmax, static_cast<uint32_t>(__shfl_xor(static_cast<int>(kmax), o)));
+  }
+  if (force_last && base_out) beat = wave_sum_int(beat);
+  for (int b = 4 * lane; b < kCdfBins; b += 256) *reinterpret_cast<u32x4 *>(bins + b) = u32x4{0, 0, 0, 0};
+  kmin = __builtin_amdgcn_readfirstlane(kmin);
+  kpos = __builtin_amdgcn_readfirstlane(kpos);
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+
+  // bucket of a key: 0 the largest; positive keys in [0, kCdfBins - 1), the others in the last
+  const uint32_t range = kmax > kpos ? kmax - kpos : 0u;
+  int sh = range ? 32 - __builtin_clz(range) - 10 : 0;  // (range >> sh) < 1024
+  sh = sh > 0 ? sh : 0;
+  if ((range >> sh) >= static_cast<uint32_t>(kCdfBins - 1)) ++sh;
+  auto bucket = [&](uint32_t k) { return k > kZero ? (kmax - k) >> sh : static_cast<uint32_t>(kCdfBins - 1); };
+  __syncthreads();
+  uint32_t slot[EPT];
+#pragma unroll
+  for (int m = 0; m < EPT; ++m) slot[m] = lane + 64 * m < K ? atomicAdd(&bins[bucket(key[m])], 1u) : 0u;
+  __syncthreads();
+  // exclusive scan, kOwn bins a thread; the largest bucket that needs an order
+  // (a bucket one key wide does not, nor does the last one while it holds zeros only)
+  const bool negative = kmin < kZero;
+  uint32_t own[kOwn], sum = 0u, big = 0u;
+#pragma unroll
+  for (int b = 0; b < kOwn; ++b) {
+    own[b] = bins[lane * kOwn + b];
+    sum += own[b];
+    if (lane == 63 && b == kOwn - 1 ? negative : sh > 0) big = max(big, own[b]);
+  }
+  uint32_t before = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = static_cast<uint32_t>(__shfl_up(static_cast<int>(before), o));
+    if (lane >= o) before += t;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) big = max(big, static_cast<uint32_t>(__shfl_xor(static_cast<int>(big), o)));
+  before -= sum;
+#pragma unroll
+  for (int b = 0; b < kOwn; ++b) {
+    bins[lane * kOwn + b] = before;
+    before += own[b];
+  }
+  if (lane == 0) bins[kCdfBins] = static_cast<uint32_t>(K);
+  __syncthreads();
+  float *fin = reinterpret_cast<float *>(buf);
+  if (__builtin_amdgcn_readfirstlane(static_cast<int>(big)) <= kBigBucket) {
+#pragma unroll
+    for (int m = 0; m < EPT; ++m)
+      if (lane + 64 * m < K) buf[bins[bucket(key[m])] + slot[m]] = key[m];
+    __syncthreads();
+    // position lane + 64 m of the grouped keys and its place (slot)
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+      const uint32_t pos = lane + 64 * m;
+      if (pos >= static_cast<uint32_t>(K)) break;
+      const uint32_t k = buf[pos];
+      const uint32_t b = bucket(k), lo = bins[b], hi = bins[b + 1];
+      uint32_t at = pos;
+      if (hi - lo > 1 && (b == kCdfBins - 1 ? negative : sh > 0)) {
+        at = lo;
+        for (uint32_t q = lo; q < hi; ++q) at += buf[q] > (q < pos ? k - 1u : k) ? 1u : 0u;  // equal keys as they lie
+      }
+      key[m] = k;
+      slot[m] = at;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < EPT; ++m)
+      if (lane + 64 * m < K) fin[slot[m]] = key_value(key[m]);
+  } else {
+    int n2 = 64;
+    while (n2 < K) n2 <<= 1;
+#pragma unroll
+    for (int m = 0; m < EPT; ++m)
+      if (lane + 64 * m < K) buf[lane + 64 * m] = key[m];
+    for (int k = K + lane; k < n2; k += 64) buf[k] = 0u;
+    for (int size = 2; size <= n2; size <<= 1) {
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        __syncthreads();
+        for (int t = lane; t < (n2 >> 1); t += 64) {
+          const int a = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), b = a + stride;  // stride: a power of two
+          const uint32_t x = buf[a], y = buf[b];
+          const bool desc = (a & size) == 0;
+          if (desc ? x < y : x > y) {
+            buf[a] = y;
+            buf[b] = x;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    for (int k = lane; k < K; k += 64) fin[k] = key_value(buf[k]);
+  }
+  __syncthreads();
+
+  // this lane's stretch
+  float v[kC];
+  bool plain = true;  // finite, not negative
+#pragma unroll
+  for (int j = 0; j < kC; ++j) {
+    const int at = kC * lane + j;
+    v[j] = at < K ? fin[at] : 0.f;
+    plain = plain && __float_as_uint(v[j]) < 0x7f800000u;
+  }
+  const uint64_t plain_lanes = __builtin_amdgcn_ballot_w64(plain);
+  const float T = thr[(row / Q) % H];
+  const int nl = (K + kC - 1) / kC;  // stretches
+  float S = 0.f;
+  int n = K, pos = 0;
+  while (pos < nl) {
+    const int e = static_cast<int>((__float_as_uint(S) >> 23) & 0xffu) - 127;
+    const int x0 = static_cast<int>((__float_as_uint(fin[kC * pos]) >> 23) & 0xffu) - 127;
+    if (S > 0.f && e >= -60 && e <= 60 && e - x0 >= kCdfTieGap) {
+      const float up = __uint_as_float(static_cast<uint32_t>(127 + 23 - e) << 23);
+      const float down = __uint_as_float(static_cast<uint32_t>(127 - 23 + e) << 23);
+      float add = 0.f;  // in units of 2^(e - 23): exact below 2^24
+      bool stop = !plain;
+#pragma unroll
+      for (int j = 0; j < kC; ++j) {
+        const float x = v[j] * up, r = __builtin_rintf(x);
+        stop = stop || __builtin_fabsf(x - r) == 0.5f;
+        add += r;
+      }
+      float incl = lane >= pos ? add : 0.f;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const float t = __shfl_up(incl, o);
+        if (lane >= o) incl += t;
+      }
+      const float tot = S * up + incl;
+      stop = stop || !(tot < 16777216.f) || !(tot * down <= T);
+      const uint64_t at = __builtin_amdgcn_ballot_w64(stop && lane >= pos && lane < nl);
+      if (at == 0) break;  // the whole row stays within T
+      const int L = __builtin_ctzll(at);
+      if (L > pos) {
+        S = __shfl(tot, L - 1) * down;
+        pos = L;
+      }
+    }
+    // stretch pos one by one; its sums only grow while it is plain, so the
+    // last one tells whether all are within T
+    float end = S;
+#pragma unroll
+    for (int j = 0; j < kC; ++j) end = end + (kC * pos + j < K ? fin[kC * pos + j] : 0.f);
+    if (!((plain_lanes >> pos) & 1) || !(end <= T)) {
+      int kept = 0;
+      bool go = true;
+      end = S;
+      for (int j = 0; j < kC && kC * pos + j < K; ++j) {
+        end = end + fin[kC * pos + j];
+        go = go && end <= T;
+        kept += go ? 1 : 0;
+      }
+      if (!go) {
+        n = kC * pos + kept;
+        break;
+      }
+    }
+    S = end;
+    ++pos;
+  }
+  if (lane == 0) {
+    n = n > min_count ? n : min_count;
+    n = n == 0 ? 1 : (n > K ? K : n);
+    count_out[row] = n;
+    if (base_out) base_out[row] = n + ((force_last && n < K && beat >= n) ? 1 : 0);
+  }
+}
+
+// The same count for rows of 2049 to 4096 key blocks, with the row sorted by rocPRIM's LDS block radix sort (256
 // threads, kItems keys each; 8-bit digits, four passes over 32-bit keys)
 // instead of the bitonic network, which costs O(K log^2 K) compare-exchanges
 // with a barrier per stage. Keys load lane-strided (coalesced), padding keys
@@ -2465,15 +2697,18 @@ extern "C" int vasc_cdf_counts(const float *score, int64_t B, int64_t H, int64_t
   const dim3 grid(static_cast<unsigned>(B * H * Q));
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int Ki = static_cast<int>(K);
-  if (K <= 256 * 16) {
-    // rows of up to 4096 key blocks: the radix-sorted count
-    auto kern = K <= 256 ? cdf_count_radix_kernel<1>
-                : K <= 512 ? cdf_count_radix_kernel<2>
-                : K <= 1024 ? cdf_count_radix_kernel<4>
-                : K <= 2048 ? cdf_count_radix_kernel<8>
-                : cdf_count_radix_kernel<16>;
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, score, H, Q, Ki, thresholds, min_count, force_last, count_out,
+  if (K <= 64 * 32) {
+    auto kern = K <= 64 * 4    ? cdf_count_rows_kernel<4>
+                : K <= 64 * 9  ? cdf_count_rows_kernel<9>
+                : K <= 64 * 17 ? cdf_count_rows_kernel<17>
+                               : cdf_count_rows_kernel<32>;
+    hipLaunchKernelGGL(kern, grid, dim3(64), 0, st, score, H, Q, Ki, thresholds, min_count, force_last, count_out,
                        base_out);
+    return check_launch("vasc_cdf_counts");
+  }
+  if (K <= 256 * 16) {
+    hipLaunchKernelGGL(cdf_count_radix_kernel<16>, grid, dim3(256), 0, st, score, H, Q, Ki, thresholds, min_count,
+                       force_last, count_out, base_out);
     return check_launch("vasc_cdf_counts");
   }
   int n2 = 64;

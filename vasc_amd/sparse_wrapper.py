@@ -115,7 +115,7 @@ def get_block_mask(pooled_score: torch.Tensor, sink_blocks: int, topk: int | Non
         out = ops.select_blocks(pooled_score, mode=_lib.MODE_TOPK, topk=0, row_cap=count, want_mask=True)
     else:
         out = ops.select_blocks(pooled_score, mode=_lib.MODE_TOPK, topk=t, want_mask=True)
-    mask = out["mask"].bool()
+    mask = out["mask"].view(torch.bool)
     if sink_blocks > 0:
         mask = torch.cat([mask, mask.new_ones(B, H, Q, sink_blocks)], dim=-1)
     return mask
@@ -284,7 +284,7 @@ def _routing_stats(score: torch.Tensor, out: dict, cap: torch.Tensor, base_mask:
     utilization = torch.where(consumed_total > 0, useful / consumed_total.clamp_min(1e-8),
                               torch.zeros_like(consumed_total))
     admitted = ops.select_workspace_region(out["workspace"], B, H, Q, K, _lib.WS_ADMITTED_DEBT)
-    selected = out["mask"].bool()
+    selected = out["mask"].view(torch.bool)
     denominator = cap.clamp_min(1).float()
     overlap = (selected & base_mask).sum(dim=-1).float()
     stats = {
@@ -317,7 +317,7 @@ def _routing_stats(score: torch.Tensor, out: dict, cap: torch.Tensor, base_mask:
             debt_priority = debt_priority.masked_fill(protected_mask.bool(), torch.finfo(torch.float32).max)
         deb = ops.select_blocks(debt_priority, mode=_lib.MODE_TOPK, topk=0, row_cap=torch.clamp(cap, max=M),
                                 max_capacity=M, want_mask=True)
-        both = (cur["mask"].bool() & deb["mask"].bool()).sum(dim=-1).float()
+        both = (cur["mask"].view(torch.bool) & deb["mask"].view(torch.bool)).sum(dim=-1).float()
         stats["cosa_pair_current_debt_overlap"] = (both / denominator).mean()
         stats["cosa_pair_history_swap_fraction"] = (1.0 - both / denominator).mean()
     return stats
@@ -384,7 +384,7 @@ def get_cosa_value_risk_pair_debt_mask(pooled_score: torch.Tensor, pooled_value:
     if stats_store is not None:
         stats_store.update(_routing_stats(pooled_score, out, cap, base_mask, (debt, pending, service), innovation,
                                           protected_mask, M))
-    return out["mask"].bool()
+    return out["mask"].view(torch.bool)
 
 
 def finalize_cosa_value_risk_pair_debt(routing_state: dict | None, *, stats_store: dict | None = None) -> dict:
@@ -503,7 +503,7 @@ def _select_for_layer(key: torch.Tensor, value: torch.Tensor, pooled_score: torc
             else:
                 bm = ops.select_blocks(pooled_score, mode=_lib.MODE_TOPK, topk=t, force_last=force_last,
                                        want_mask=True)
-            base_mask = bm["mask"].bool()
+            base_mask = bm["mask"].view(torch.bool)
             protected = None
             if force_last:
                 protected = torch.zeros_like(base_mask)
