@@ -119,7 +119,8 @@ def adaptive_sparse_attention_forward(self, x: torch.Tensor, pos: torch.Tensor, 
     qkv = self.qkv(x).to(torch.bfloat16).view(B, NP, 3, nh, hd)
     rope = getattr(self, "rope", None)
     n_patch = N * (P - S)
-    vasc_mode = routing_config().mode == "vasc"
+    cfg = routing_config()  # the environment's switches, read once for the layer
+    vasc_mode = cfg.mode == "vasc"
     if pool_mode == "avg" and n_patch > 0 and fused_layout_supported(self):
         # layout, V tiles, block means and value innovation in one pass
         tables = rope.tables(hd, x.device) if rope is not None else None
@@ -135,7 +136,7 @@ def adaptive_sparse_attention_forward(self, x: torch.Tensor, pos: torch.Tensor, 
             q_patch, q_special, k_re, None, attn_pooled, sparse_ratio=sparse_ratio, cdf_threshold=cdf_threshold,
             layer_idx=layer_idx, routing_state=routing_state, num_patch_tokens=n_patch,
             want_sparsity=aux_output_store is not None, _innovation=innovation, token_layout=(N, P, S), _vt=vt,
-            _priority=priority, _scale=ops.LN2, **research)
+            _priority=priority, _scale=ops.LN2, _cfg=cfg, **research)
         return _finish(self, x, tokens_out, sparsity, aux_output_store)
     if fused_layout_supported(self):
         tables = rope.tables(hd, x.device) if rope is not None else None
@@ -160,7 +161,8 @@ def adaptive_sparse_attention_forward(self, x: torch.Tensor, pos: torch.Tensor, 
     tokens_out, _, sparsity = sparse_global_attention(
         q_patch, q_special, k_re, v_re, attn_pooled, sparse_ratio=sparse_ratio, cdf_threshold=cdf_threshold,
         layer_idx=layer_idx, routing_state=routing_state, num_patch_tokens=n_patch,
-        want_sparsity=aux_output_store is not None, _innovation=innovation, token_layout=(N, P, S), **research)
+        want_sparsity=aux_output_store is not None, _innovation=innovation, token_layout=(N, P, S), _cfg=cfg,
+        **research)
     return _finish(self, x, tokens_out, sparsity, aux_output_store)
 
 

@@ -111,11 +111,18 @@ def use_mode(backbone: str, mode: str):
         os.environ.update(saved)
 
 
+_PREFIX = "SPARSE_VGGT_"
 _TRUE = {"1", "true", "yes", "on"}
+# Switches of research routers that this build does not implement.
+_RESEARCH_SWITCHES = tuple(_PREFIX + n for n in (
+    "COSA_ORDERED_LUT", "COSA_TOPK_ORDERED_LUT", "COSA_COMPACT_ORDERED_LUT", "COSA_HRM_ORDERED_LUT",
+    "COSA_KERNEL_PAIR_SERVICE", "PROJECTED_QK_DEBT", "PROJECTED_QK_PV_DEBT", "COSA_BUDGET_ONLY_UPSTREAM",
+    "COSA_UNIFORM_CAPACITY_HINT", "COSA_RISK_SAFE_OBSERVER", "QK_VALUE_RISK_OBSERVER", "QK_BUNDLE_OBSERVER",
+    "COLLECT_QK_PV_SERVICE", "RADIAL_A_DENSE", "RADIAL_A_CHUNKED"))
 
 
 def _flag(env, name: str, default: str = "0") -> bool:
-    return env.get("SPARSE_VGGT_" + name, default).lower() in _TRUE
+    return env.get(_PREFIX + name, default).lower() in _TRUE
 
 
 @dataclass(frozen=True)
@@ -138,12 +145,7 @@ def routing_config(env=None) -> RoutingConfig:
     """
     env = os.environ if env is None else env
     vasc = _flag(env, "COSA_VALUE_RISK_PAIR_DEBT")
-    unsupported = [n for n in ("COSA_ORDERED_LUT", "COSA_TOPK_ORDERED_LUT", "COSA_COMPACT_ORDERED_LUT",
-                               "COSA_HRM_ORDERED_LUT", "COSA_KERNEL_PAIR_SERVICE", "PROJECTED_QK_DEBT",
-                               "PROJECTED_QK_PV_DEBT", "COSA_BUDGET_ONLY_UPSTREAM", "COSA_UNIFORM_CAPACITY_HINT",
-                               "COSA_RISK_SAFE_OBSERVER", "QK_VALUE_RISK_OBSERVER", "QK_BUNDLE_OBSERVER",
-                               "COLLECT_QK_PV_SERVICE", "RADIAL_A_DENSE", "RADIAL_A_CHUNKED")
-                   if _flag(env, n)]
+    unsupported = [n[len(_PREFIX):] for n in _RESEARCH_SWITCHES if env.get(n, "0").lower() in _TRUE]
     domain = "qk_admission"
     if vasc:
         domain = env.get("SPARSE_VGGT_COSA_DEBT_SERVICE_DOMAIN", "pv_execution").lower()
@@ -154,7 +156,7 @@ def routing_config(env=None) -> RoutingConfig:
         if not _flag(env, "COSA_CONSERVATIVE_DEBT_PROJECTION"):
             unsupported.append("COSA_CONSERVATIVE_DEBT_PROJECTION=0")
     threshold = env.get("SPARSE_VGGT_QK_PV_THRESHOLD", "1e10")
-    if threshold != "sequence_mass_bound":
+    if threshold not in ("sequence_mass_bound", "1e10"):
         try:
             resolve_pv_threshold(threshold, 2)
         except ValueError as exc:

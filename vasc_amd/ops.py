@@ -22,7 +22,8 @@ LOG2E, LN2 = 1.4426950408889634, 0.6931471805599453
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without the two Python objects
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t: torch.Tensor, name: str) -> None:

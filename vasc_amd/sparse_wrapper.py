@@ -32,7 +32,7 @@ import os
 import torch
 
 from . import _lib, ops
-from .launcher import pv_threshold_active, resolve_pv_threshold, routing_config
+from .launcher import RoutingConfig, pv_threshold_active, resolve_pv_threshold, routing_config
 
 KBLK = 64
 STATE_KEY = "cosa_value_risk_pair_debt"
@@ -245,10 +245,9 @@ def _record_pv_execution(routing_state: dict | None, pv_map: torch.Tensor | None
     }
 
 
-def _pv_threshold(key: torch.Tensor, layer_idx: int) -> float | None:
+def _pv_threshold(key: torch.Tensor, layer_idx: int, cfg: RoutingConfig) -> float | None:
     """The PV post-cut threshold of this layer (SW:7008-7027), or None when
     it is inert (1e10, or the layer is not in QK_PV_ACTIVE_LAYERS)."""
-    cfg = routing_config()
     thr = resolve_pv_threshold(cfg.pv_threshold, key.shape[-2])
     if not pv_threshold_active(cfg.pv_active_layers, layer_idx) or thr >= 1e10:
         return None
@@ -443,7 +442,7 @@ def _check_research_kwargs(kwargs: dict) -> None:
 
 def _select_for_layer(key: torch.Tensor, value: torch.Tensor, pooled_score: torch.Tensor, topk, sparse_ratio,
                       cdf_threshold, layer_idx: int, routing_stats_store, routing_state, num_patch_tokens,
-                      research: dict, innovation: torch.Tensor | None = None,
+                      research: dict, cfg: RoutingConfig, innovation: torch.Tensor | None = None,
                       priority: torch.Tensor | None = None):
     """Mode switch, budget, mixed-tail and sink rules and kernel 2 of
     block_sparse_attn_cuda (SW:6998-7041, 7559-7770). Returns the selection
@@ -454,7 +453,6 @@ def _select_for_layer(key: torch.Tensor, value: torch.Tensor, pooled_score: torc
     for t, name in ((key, "key"), (value, "value"), (pooled_score, "pooled_score")):
         if t is not None:
             _require_gpu(t, name)
-    cfg = routing_config()
     Tk = key.shape[-2]
     orig_kblk = pooled_score.shape[-1]
     total_kblk = math.ceil(Tk / KBLK)
@@ -547,9 +545,10 @@ def block_sparse_attn_cuda(query: torch.Tensor, key: torch.Tensor, value: torch.
     in bf16. Returns ``o`` (query dtype) or ``(o, sparsity)``.
     """
     _require_gpu(query, "query")
+    cfg = routing_config()
     sel, total_kblk = _select_for_layer(key, value, pooled_score, topk, sparse_ratio, cdf_threshold, layer_idx,
-                                        routing_stats_store, routing_state, num_patch_tokens, research)
-    thr = _pv_threshold(key, layer_idx)
+                                        routing_stats_store, routing_state, num_patch_tokens, research, cfg)
+    thr = _pv_threshold(key, layer_idx, cfg)
     if key.dtype == value.dtype == torch.float16 and key.shape == value.shape:
         key, vt = ops.pack_kv_half(key, value)  # one pass over both
     else:
@@ -574,7 +573,7 @@ def sparse_global_attention(q_patch: torch.Tensor, q_special: torch.Tensor | Non
                             num_patch_tokens: int | None = None, want_sparsity: bool = True,
                             _innovation: torch.Tensor | None = None, token_layout: tuple | None = None,
                             _vt: torch.Tensor | None = None, _priority: torch.Tensor | None = None,
-                            _scale: float | None = None, **research):
+                            _scale: float | None = None, _cfg: RoutingConfig | None = None, **research):
     """``block_sparse_attn_cuda`` for a whole global layer: the selection of
     the patch queries as there, and the special-token queries (which the
     reference runs through a dense SDPA, ATT:8464-8484) over every key in
@@ -588,15 +587,17 @@ def sparse_global_attention(q_patch: torch.Tensor, q_special: torch.Tensor | Non
     ``value`` may be None); ``_priority``: ``pooled_score`` cleaned as the
     ledger stores it (``ops.pooled_softmax(..., priority=True)``);
     ``_scale``: the softmax scale where it is not ``D ** -0.5`` (``ops.LN2``
-    for queries packed with theirs)."""
+    for queries packed with theirs); ``_cfg``: the ``routing_config()`` that
+    the caller read for this call."""
     _require_gpu(q_patch, "query")
     if value is None and _vt is None:
         raise ValueError("sparse_global_attention requires the values (or their packed tiles)")
+    cfg = routing_config() if _cfg is None else _cfg
     sel, total_kblk = _select_for_layer(key, value, pooled_score, topk, sparse_ratio, cdf_threshold, layer_idx,
-                                        routing_stats_store, routing_state, num_patch_tokens, research,
+                                        routing_stats_store, routing_state, num_patch_tokens, research, cfg,
                                         innovation=_innovation, priority=_priority)
     vt = ops.pack_v(value) if _vt is None else _vt
-    thr = _pv_threshold(key, layer_idx)
+    thr = _pv_threshold(key, layer_idx, cfg)
     if thr is None:
         if token_layout is not None:
             out = ops.global_attn_tokens(q_patch, q_special, key, vt, sel["index"], sel["count"], *token_layout,
