@@ -480,6 +480,37 @@ int vasc_restore_tokens(const uint16_t *x_patch, int64_t p_sb, int64_t p_sh,
                         int64_t N, int64_t P, int64_t S, int64_t d,
                         uint16_t *out, void *stream);
 
+/* vasc_global_attn_fwd and vasc_global_attn_tokens_fwd with a workspace (16-byte
+ * aligned) in which the special queries' keys may be split over several workgroups.
+ * vasc_global_attn_workspace_size: its bytes, 0 where no split is made (then it
+ * may be NULL). */
+int64_t vasc_global_attn_workspace_size(int64_t B, int64_t H, int64_t n_patch, int64_t n_special,
+                                        int64_t nk, int64_t index_width);
+int vasc_global_attn_ws_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh,
+                         int64_t qp_st, const uint16_t *q_special,
+                         int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                         const uint16_t *k, int64_t k_sb, int64_t k_sh,
+                         int64_t k_st, const uint16_t *vt, uint16_t *o_patch,
+                         int64_t op_sb, int64_t op_sh, int64_t op_st,
+                         uint16_t *o_special, int64_t os_sb, int64_t os_sh,
+                         int64_t os_st, int64_t B, int64_t H, int64_t n_patch,
+                         int64_t n_special, int64_t nk, int64_t d,
+                         const int32_t *block_index, int64_t index_width,
+                         const int32_t *block_count, float sm_scale,
+                         void *workspace, int64_t workspace_bytes, void *stream);
+int vasc_global_attn_tokens_ws_fwd(const uint16_t *q_patch, int64_t qp_sb,
+                                int64_t qp_sh, int64_t qp_st,
+                                const uint16_t *q_special, int64_t qs_sb,
+                                int64_t qs_sh, int64_t qs_st,
+                                const uint16_t *k, int64_t k_sb, int64_t k_sh,
+                                int64_t k_st, const uint16_t *vt,
+                                uint16_t *out, int64_t B, int64_t H, int64_t N,
+                                int64_t P, int64_t S, int64_t nk, int64_t d,
+                                const int32_t *block_index,
+                                int64_t index_width,
+                                const int32_t *block_count, float sm_scale,
+                                void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Operator inputs in IEEE half (the reference's dtype), rounded to bf16 as they
  * are read: vasc_pool_qkv with every given tensor in half; V packed as
  * vasc_pack_v and, with k, K as contiguous bf16 [B,H,nk,d] in the same pass;

@@ -251,6 +251,44 @@ def test_prescaled_queries_match_the_oracle(N, P, S, H):
     _check(patch, rows)
 
 
+@pytest.mark.parametrize("level", [None, "high", "low"])
+@pytest.mark.parametrize("N,P,S,parts", [(1, 4032, 1, 1), (1, 4033, 5, 2), (3, 1409, 45, 2), (2, 4099, 65, 4),
+                                         (1, 16391, 129, 8)])
+def test_split_special_queries_match_the_oracle(N, P, S, parts, level):
+    """Special queries whose keys are split over workgroups, at part counts 1,
+    2, 4 and 8, ragged last parts and a second query block. "high": the first
+    key block's logits near 2^150, "low": the last part's all near 2^-160; both
+    are out of the sums' range and take the second walk. The file's tolerance:
+    the parts only change the order of a float32 addition."""
+    from vasc_amd import _lib, ops
+    H, nk, n_patch, n_sp = 2, N * P, N * (P - S), N * S
+    nkb = math.ceil(nk / 64)
+    q, k, v = _rand((1, H, nk, 64), 50), _rand((1, H, nk, 64), 51), _rand((1, H, nk, 64), 52)
+    if level is not None:  # q0 * k0 / 8 * log2(e) = 150 or -160
+        q[..., 0] = 8.0
+        k[..., 0] = 0.0
+        if level == "high":
+            k[:, :, :64, 0] = 150.0 / math.log2(math.e)
+        else:
+            k[:, :, (parts - 1) * math.ceil(nkb / parts) * 64:, 0] = -160.0 / math.log2(math.e)
+    qp, qs, kc, vt = q[:, :, :n_patch].cuda(), q[:, :, n_patch:].cuda(), k.cuda(), ops.pack_v(v.cuda())
+    idx = torch.zeros(1, H, math.ceil(n_patch / 128), 1, dtype=torch.int32)
+    cnt = torch.ones(1, H, math.ceil(n_patch / 128), dtype=torch.int32)
+    size = _lib.fn("vasc_global_attn_workspace_size")(1, H, n_patch, n_sp, nk, 1)
+    assert size == (0 if parts == 1 else H * math.ceil(n_sp / 128) * parts * 128 * 65 * 4)
+    full = torch.arange(nkb, dtype=torch.int32).expand(1, H, math.ceil(n_sp / 128), nkb).contiguous()
+    ref = OA.block_sparse_attention(q[:, :, n_patch:].float().numpy(), k.float().numpy(), v.float().numpy(), full.numpy(),
+                                    torch.full(full.shape[:3], nkb, dtype=torch.int32).numpy())
+    refp = OA.block_sparse_attention(q[:, :, :n_patch].float().numpy(), k.float().numpy(), v.float().numpy(), idx.numpy(),
+                                     cnt.numpy())
+    op, os_ = ops.global_attn(qp, qs, kc, vt, idx.cuda(), cnt.cuda())
+    _check(os_, ref)
+    _check(op, refp)
+    out = ops.global_attn_tokens(qp, qs, kc, vt, idx.cuda(), cnt.cuda(), N, P, S).view(1, N, P, H, 64)
+    assert torch.equal(out[:, :, :S].reshape(1, n_sp, H, 64).transpose(1, 2), os_)
+    assert torch.equal(out[:, :, S:].reshape(1, n_patch, H, 64).transpose(1, 2), op)
+
+
 # ---------------------------------------------------------------- PV post-cut
 def _graded_blocks(nq, nk, levels, seed):
     """Query rows a*e0 (+ small noise) and key block j = levels[j] / c * e0

@@ -37,6 +37,7 @@ SIGNATURES: dict[str, tuple] = {
                                 I64, I64, I64, I64, I64, I64, I64, P, P, P, P, P]),
     "vasc_pooled_softmax": (c_int32, [P, P, I64, I64, I64, I64, I64, c_float, I32, P, P, P, P]),
     "vasc_pooled_softmax_workspace_size": (I64, [I64, I64, I64, I64]),
+    "vasc_global_attn_workspace_size": (I64, [I64, I64, I64, I64, I64, I64]),
     "vasc_pair_innovation": (c_int32, [P, I64, I64, I64, I64, P, P]),
     "vasc_select_workspace_size": (c_size_t, [I64, I64, I64, I64]),
     "vasc_select_workspace_offset": (I64, [I64, I64, I64, I64, I32]),
@@ -61,8 +62,13 @@ SIGNATURES: dict[str, tuple] = {
     "vasc_global_attn_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64, P,
                                        P, I64, I64, I64, P, I64, I64, I64, I64, I64, I64, I64, I64, I64,
                                        P, I64, P, c_float, P]),
+    "vasc_global_attn_ws_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64, P,
+                                       P, I64, I64, I64, P, I64, I64, I64, I64, I64, I64, I64, I64, I64,
+                                       P, I64, P, c_float, P, I64, P]),
     "vasc_global_attn_tokens_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64, P, P,
                                               I64, I64, I64, I64, I64, I64, I64, P, I64, P, c_float, P]),
+    "vasc_global_attn_tokens_ws_fwd": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64, P, P,
+                                              I64, I64, I64, I64, I64, I64, I64, P, I64, P, c_float, P, I64, P]),
     "vasc_pack_qkv": (c_int32, [P, I64, I64, I64, P, I64, I64, I64, P, I64, I64, I64,
                                 I64, I64, I64, I64, I64, I64, P, P, c_float, I32, P, P, c_float, I32,
                                 P, I64, I64, P, P, I64, P, P, P, P, P]),

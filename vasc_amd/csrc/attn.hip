@@ -103,6 +103,11 @@ struct AttnParams {
   const float *pv_thr;
   int32_t *pv_map;
   int64_t pv_w;
+  // key split of the special queries: nsplit workgroups walk split_blocks key
+  // blocks each and leave float32 partial results, [num_wg2][nsplit][128 rows]
+  // of 64 sums of P V, then of the row sums
+  int32_t nsplit, split_blocks;
+  float *part;
 };
 
 __device__ __forceinline__ floatx16 mfma32(u32x4 a, u32x4 b, floatx16 c) {
@@ -334,7 +339,7 @@ __device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_a
 // them), so the probabilities are exp2(S) without a product per score: 690
 // cycles a wave-block against 770 and 1.00 ms against 1.06 on lists of 132 of
 // 521 blocks, 16 heads.
-template <bool kDense, bool kUnit>
+template <bool kDense, bool kUnit, bool kSplit>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void bsattn_fwd_kernel(const AttnParams p) {
   constexpr int CH = 512 / kThreads;  // 16-byte chunks per thread per tile
@@ -350,9 +355,12 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const int64_t hw = dense && !kDense ? static_cast<int64_t>(blockIdx.x)
                                       : static_cast<int64_t>(blockIdx.x) - p.num_wg2_slots;
   const int64_t wg = p.head_major ? hw : xcd_remap(hw, dense && !kDense ? p.num_wg2_slots : p.num_wg);
-  if (dense && !kDense && wg >= p.num_wg2) return;  // padding of the special-query slots
-  const int qb = static_cast<int>(wg % nqb);
-  const int64_t bh = wg / nqb;
+  const bool sp = dense && !kDense;  // a special-query workgroup
+  if (sp && wg >= p.num_wg2 * (kSplit ? p.nsplit : 1)) return;  // padding of the special-query slots
+  const int64_t unit = kSplit && sp ? wg / p.nsplit : wg;
+  const int split = kSplit && sp ? static_cast<int>(wg % p.nsplit) : 0;
+  const int qb = static_cast<int>(unit % nqb);
+  const int64_t bh = unit / nqb;
   const int64_t h = bh % p.H;
   const int64_t b = bh / p.H;
   const int tid = threadIdx.x;
@@ -361,8 +369,10 @@ void bsattn_fwd_kernel(const AttnParams p) {
 
   int n;
   const int32_t *list = nullptr;
+  const int blk0 = kSplit && sp ? split * p.split_blocks : 0;  // first block of a dense walk
   if (dense) {
-    n = static_cast<int>(p.nkb);
+    n = static_cast<int>(p.nkb) - blk0;
+    if (kSplit && sp && n > p.split_blocks) n = p.split_blocks;
   } else {
     const int64_t row = bh * p.nqb + qb;
     list = p.idx + row * p.idx_w;
@@ -370,7 +380,6 @@ void bsattn_fwd_kernel(const AttnParams p) {
     n = n < 0 ? 0 : (n > p.idx_w ? static_cast<int>(p.idx_w) : n);
   }
 
-  const bool sp = dense && !kDense;  // a special-query workgroup
   const uint16_t *qsrc = sp ? p.q2 : p.q;
   const int64_t q_sb = sp ? p.q2_sb : p.q_sb, q_sh = sp ? p.q2_sh : p.q_sh, q_st = sp ? p.q2_st : p.q_st;
   const int64_t nq = sp ? p.nq2 : p.nq;
@@ -549,7 +558,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   // share of the tiles and keeps the barriers.
   auto walk = [&](auto idle_wave) __attribute__((always_inline)) {
     constexpr bool kIdle = decltype(idle_wave)::value;
-    int blk = dense ? 0 : clist[0];
+    int blk = dense ? blk0 : clist[0];
     int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
     fetch(blk, 0);
     int nw = n;
@@ -560,7 +569,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
       const int lim = valid_keys(blk);
       if (j + 1 < nw) {
         if (dense) {
-          blk = j + 1;
+          ++blk;
         } else {
           const int e = e_next;
           blk = p.delta ? blk + e : e;
@@ -603,12 +612,78 @@ void bsattn_fwd_kernel(const AttnParams p) {
     }
   }
 
-  store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
+  if (kSplit && sp) {
+    float *part = p.part + wg * (kBlockQ * (kHeadDim + 1));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = w * 32 + 16 * i + lr;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) *reinterpret_cast<floatx4 *>(part + r * kHeadDim + 16 * t + 4 * g4) = oacc[i][t];
+      if (g4 == 0) part[kBlockQ * kHeadDim + r] = lacc[i][0];
+    }
+  } else {
+    store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
+  }
   // last, so that no result lives across the call: its stores follow these
   __syncthreads();  // every wave is done with the tiles and with redo
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0))
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0)) {
+    if (kSplit && sp) {  // combine_kernel walks the rows again
+      if (tid < kBlockQ) p.part[wg * (kBlockQ * (kHeadDim + 1)) + kBlockQ * kHeadDim + tid] = -INFINITY;
+      return;
+    }
     bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()), lds0,
-                  kDense, static_cast<int>(wg), n);
+                  kDense, static_cast<int>(unit), n);
+  }
+}
+
+// Results of split special queries: the partial sums in split order, normalised
+// (thread: row tid / 2, 32 features). Rows that any part found out of range
+// are walked again, every key, with the running maximum.
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void combine_kernel(const AttnParams p) {
+  __shared__ __attribute__((aligned(16))) uint16_t tiles[2][kTile];
+  const int64_t unit = blockIdx.x;
+  const int64_t bh = unit / p.nq2b, h = bh % p.H, b = bh / p.H;
+  const int r = threadIdx.x >> 1, d0 = (threadIdx.x & 1) * 32;
+  const int64_t qrow = (unit % p.nq2b) * kBlockQ + r;
+  floatx4 acc[8];
+  float l = 0.f;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  if (qrow < p.nq2) {
+    for (int s = 0; s < p.nsplit; ++s) {
+      const float *part = p.part + (unit * p.nsplit + s) * (kBlockQ * (kHeadDim + 1));
+      l += part[kBlockQ * kHeadDim + r];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const floatx4 o = *reinterpret_cast<const floatx4 *>(part + r * kHeadDim + d0 + 4 * c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[c][e] += o[e];
+      }
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    uint16_t *optr = p.o2 + b * p.o2_sb + h * p.o2_sh +
+                     (p.tok_p > 0 ? (qrow / p.tok_s) * p.tok_p + qrow % p.tok_s : qrow) * p.o2_st + d0;
+#pragma unroll
+    for (int c = 0; c < 8; c += 2) {
+      const u32x4 v = {pack_bf16x2(acc[c][0] * inv, acc[c][1] * inv), pack_bf16x2(acc[c][2] * inv, acc[c][3] * inv),
+                       pack_bf16x2(acc[c + 1][0] * inv, acc[c + 1][1] * inv),
+                       pack_bf16x2(acc[c + 1][2] * inv, acc[c + 1][3] * inv)};
+      *reinterpret_cast<u32x4 *>(optr + 4 * c) = v;
+    }
+  }
+  // out of range, marked -inf by a part (weights are never negative), or a sum
+  // of finite parts past the float range
+  bool bad = __float_as_uint(l) - kLowBits > kHighBits - kLowBits;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bad |= (__float_as_uint(acc[c][e]) & 0x7fffffffu) >= 0x7f800000u;
+  bad = bad && qrow < p.nq2;
+  __syncthreads();  // these stores come before those of the second walk
+  if (__syncthreads_or(bad))
+    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()),
+                  lds_addr32(tiles), false, static_cast<int>(unit), static_cast<int>(p.nkb));
 }
 
 // The PV post-cut (qk_int_sv_f16_cuda_sm80.cuh:291-381): 4 waves x 32 query
@@ -916,6 +991,24 @@ struct OutTokens {
   int64_t P = 0, S = 0;
 };
 
+// How many workgroups share a special-query block's keys. Such a block walks
+// every key block while a patch block walks its list (index_w entries), and the
+// patch blocks keep the card (1024 resident workgroups) busy for about
+// index_w * max(1, num_wg / 1024) of these steps: the special blocks are split to
+// end with them, into parts of at least 32 key blocks. Below 64 blocks the second
+// launch and the workspace cost the host more than the split saves: at 2 frames of
+// 1041 tokens the launch fell from 29 to 24 us and the layer, bound by the host,
+// rose from 421 to 435. To the nearest part count: two parts for a walk that
+// already ends with the patch blocks cost the 32-frame layer 0.4 to 1.1%. Unsplit,
+// patch blocks alone and split, 16 heads, lists of a quarter: 56, 30 and 39 us at
+// 4 frames; 120, 89 and 97 at 8; 300, 289 and 296 at 16.
+int64_t special_splits(int64_t num_wg, int64_t nkb, int64_t index_w) {
+  const int64_t busy = index_w * (num_wg > 1024 ? num_wg : 1024) / 1024;
+  int64_t n = busy > 0 ? (nkb + busy / 2) / busy : 1;
+  if (n > nkb / 32) n = nkb / 32;
+  return n < 1 ? 1 : (n > 8 ? 8 : n);
+}
+
 // Special-token queries of vasc_global_attn_fwd (absent: q2 == NULL).
 struct SpecialQueries {
   const uint16_t *q2 = nullptr;
@@ -923,6 +1016,7 @@ struct SpecialQueries {
   uint16_t *o2 = nullptr;
   int64_t o2_sb = 0, o2_sh = 0, o2_st = 0;
   int64_t nq2 = 0;
+  float *part = nullptr;  // workspace of the key split (absent: no split)
 };
 
 int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64_t q_st,
@@ -960,7 +1054,11 @@ int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64
   p.nq2 = sq.q2 ? sq.nq2 : 0;
   p.nq2b = cdiv(p.nq2, kBlockQ);
   p.num_wg2 = B * H * p.nq2b;
-  p.num_wg2_slots = (p.num_wg2 + 7) / 8 * 8;
+  const int64_t nsplit = p.num_wg2 && sq.part ? special_splits(p.num_wg, p.nkb, idx_w) : 1;
+  p.nsplit = static_cast<int32_t>(nsplit);
+  p.split_blocks = static_cast<int32_t>(cdiv(p.nkb, nsplit));
+  p.part = sq.part;
+  p.num_wg2_slots = (p.num_wg2 * nsplit + 7) / 8 * 8;
   // K and V of one head take 256 B per key token; from 192k tokens (48 MB a
   // head) the eight heads one per XCD that the contiguous mapping keeps in
   // flight exceed the 256 MB Infinity Cache by half, and walking the heads
@@ -978,11 +1076,15 @@ int launch_attn(bool dense, const uint16_t *q, int64_t q_sb, int64_t q_sh, int64
   p.half_io = half_io ? 1 : 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   auto kern = pv_thr ? bsattn_pv_kernel
-              : dense      ? bsattn_fwd_kernel<true, false>
-              : p.c == 1.f ? bsattn_fwd_kernel<false, true>
-                           : bsattn_fwd_kernel<false, false>;
+              : dense      ? bsattn_fwd_kernel<true, false, false>
+              : p.c == 1.f ? bsattn_fwd_kernel<false, true, false>
+                           : bsattn_fwd_kernel<false, false, false>;
+  if (nsplit > 1) kern = p.c == 1.f ? bsattn_fwd_kernel<false, true, true> : bsattn_fwd_kernel<false, false, true>;
   hipLaunchKernelGGL(kern, dim3(p.num_wg + p.num_wg2_slots), dim3(kThreads), 0, s, p);
-  return check_launch(dense ? "vasc_dense_attn_fwd" : "vasc_block_sparse_attn_fwd");
+  if ((rc = check_launch(dense ? "vasc_dense_attn_fwd" : "vasc_block_sparse_attn_fwd"))) return rc;
+  if (nsplit == 1) return VASC_OK;
+  hipLaunchKernelGGL(combine_kernel, dim3(p.num_wg2), dim3(kThreads), 0, s, p);
+  return check_launch("vasc_global_attn/combine");
 }
 
 }  // namespace
@@ -1034,14 +1136,22 @@ extern "C" int vasc_dense_attn_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh
                            nk, d, nullptr, 1, nullptr, 0, sm_scale, stream);
 }
 
-extern "C" int vasc_global_attn_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
-                                    const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
-                                    const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
-                                    const uint16_t *vt, uint16_t *o_patch, int64_t op_sb, int64_t op_sh,
-                                    int64_t op_st, uint16_t *o_special, int64_t os_sb, int64_t os_sh,
-                                    int64_t os_st, int64_t B, int64_t H, int64_t n_patch, int64_t n_special,
-                                    int64_t nk, int64_t d, const int32_t *block_index, int64_t index_width,
-                                    const int32_t *block_count, float sm_scale, void *stream) {
+extern "C" int64_t vasc_global_attn_workspace_size(int64_t B, int64_t H, int64_t n_patch, int64_t n_special, int64_t nk,
+                                                   int64_t index_width) {
+  using namespace vasc;
+  if (B <= 0 || H <= 0 || n_patch <= 0 || n_special <= 0 || nk <= 0 || index_width <= 0) return 0;
+  const int64_t n = special_splits(B * H * cdiv(n_patch, kBlockQ), cdiv(nk, kBlockK), index_width);
+  return n == 1 ? 0 : B * H * cdiv(n_special, kBlockQ) * n * kBlockQ * (kHeadDim + 1) * 4;
+}
+
+static int global_attn_impl(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                            const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                            const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t *vt,
+                            uint16_t *o_patch, int64_t op_sb, int64_t op_sh, int64_t op_st, uint16_t *o_special,
+                            int64_t os_sb, int64_t os_sh, int64_t os_st, int64_t B, int64_t H, int64_t n_patch,
+                            int64_t n_special, int64_t nk, int64_t d, const int32_t *block_index,
+                            int64_t index_width, const int32_t *block_count, float sm_scale, void *workspace,
+                            int64_t workspace_bytes, void *stream) {
   using namespace vasc;
   SpecialQueries sq;
   if (n_special > 0) {
@@ -1051,19 +1161,53 @@ extern "C" int vasc_global_attn_fwd(const uint16_t *q_patch, int64_t qp_sb, int6
     sq.q2 = q_special; sq.q2_sb = qs_sb; sq.q2_sh = qs_sh; sq.q2_st = qs_st;
     sq.o2 = o_special; sq.o2_sb = os_sb; sq.o2_sh = os_sh; sq.o2_st = os_st;
     sq.nq2 = n_special;
+    if (workspace) {
+      VASC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "workspace must be 16-byte aligned");
+      VASC_REQUIRE(workspace_bytes >= vasc_global_attn_workspace_size(B, H, n_patch, sq.nq2, nk, index_width),
+                   "workspace of %lld bytes is too small", (long long)workspace_bytes);
+      sq.part = static_cast<float *>(workspace);
+    }
   }
   VASC_REQUIRE(n_special >= 0, "n_special must be non-negative");
   return launch_attn(false, q_patch, qp_sb, qp_sh, qp_st, k, k_sb, k_sh, k_st, vt, o_patch, op_sb, op_sh, op_st,
                      B, H, n_patch, nk, d, block_index, index_width, block_count, 0, sm_scale, stream, sq);
 }
 
-extern "C" int vasc_global_attn_tokens_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
-                                           const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
-                                           const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
-                                           const uint16_t *vt, uint16_t *out, int64_t B, int64_t H, int64_t N,
-                                           int64_t P, int64_t S, int64_t nk, int64_t d,
-                                           const int32_t *block_index, int64_t index_width,
-                                           const int32_t *block_count, float sm_scale, void *stream) {
+extern "C" int vasc_global_attn_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                                    const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                                    const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                    const uint16_t *vt, uint16_t *o_patch, int64_t op_sb, int64_t op_sh,
+                                    int64_t op_st, uint16_t *o_special, int64_t os_sb, int64_t os_sh,
+                                    int64_t os_st, int64_t B, int64_t H, int64_t n_patch, int64_t n_special,
+                                    int64_t nk, int64_t d, const int32_t *block_index, int64_t index_width,
+                                    const int32_t *block_count, float sm_scale, void *stream) {
+  return global_attn_impl(q_patch, qp_sb, qp_sh, qp_st, q_special, qs_sb, qs_sh, qs_st, k, k_sb, k_sh, k_st, vt,
+                          o_patch, op_sb, op_sh, op_st, o_special, os_sb, os_sh, os_st, B, H, n_patch, n_special,
+                          nk, d, block_index, index_width, block_count, sm_scale, nullptr, 0, stream);
+}
+
+extern "C" int vasc_global_attn_ws_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                                       const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                                       const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                       const uint16_t *vt, uint16_t *o_patch, int64_t op_sb, int64_t op_sh,
+                                       int64_t op_st, uint16_t *o_special, int64_t os_sb, int64_t os_sh,
+                                       int64_t os_st, int64_t B, int64_t H, int64_t n_patch, int64_t n_special,
+                                       int64_t nk, int64_t d, const int32_t *block_index, int64_t index_width,
+                                       const int32_t *block_count, float sm_scale, void *workspace,
+                                       int64_t workspace_bytes, void *stream) {
+  return global_attn_impl(q_patch, qp_sb, qp_sh, qp_st, q_special, qs_sb, qs_sh, qs_st, k, k_sb, k_sh, k_st, vt,
+                          o_patch, op_sb, op_sh, op_st, o_special, os_sb, os_sh, os_st, B, H, n_patch, n_special,
+                          nk, d, block_index, index_width, block_count, sm_scale, workspace, workspace_bytes,
+                          stream);
+}
+
+static int global_attn_tokens_impl(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                                   const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                                   const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st, const uint16_t *vt,
+                                   uint16_t *out, int64_t B, int64_t H, int64_t N, int64_t P, int64_t S, int64_t nk,
+                                   int64_t d, const int32_t *block_index, int64_t index_width,
+                                   const int32_t *block_count, float sm_scale, void *workspace,
+                                   int64_t workspace_bytes, void *stream) {
   using namespace vasc;
   VASC_REQUIRE(N > 0 && P > S && S >= 0, "invalid frame sizes N=%lld P=%lld S=%lld", (long long)N, (long long)P,
                (long long)S);
@@ -1078,6 +1222,12 @@ extern "C" int vasc_global_attn_tokens_fwd(const uint16_t *q_patch, int64_t qp_s
     sq.q2 = q_special; sq.q2_sb = qs_sb; sq.q2_sh = qs_sh; sq.q2_st = qs_st;
     sq.o2 = out; sq.o2_sb = o_sb; sq.o2_sh = o_sh; sq.o2_st = o_st;
     sq.nq2 = N * S;
+    if (workspace) {
+      VASC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "workspace must be 16-byte aligned");
+      VASC_REQUIRE(workspace_bytes >= vasc_global_attn_workspace_size(B, H, N * (P - S), sq.nq2, nk, index_width),
+                   "workspace of %lld bytes is too small", (long long)workspace_bytes);
+      sq.part = static_cast<float *>(workspace);
+    }
   }
   OutTokens ot;
   ot.P = P;
@@ -1085,4 +1235,29 @@ extern "C" int vasc_global_attn_tokens_fwd(const uint16_t *q_patch, int64_t qp_s
   return launch_attn(false, q_patch, qp_sb, qp_sh, qp_st, k, k_sb, k_sh, k_st, vt, out, o_sb, o_sh, o_st, B, H,
                      N * (P - S), nk, d, block_index, index_width, block_count, 0, sm_scale, stream, sq, nullptr,
                      nullptr, ot);
+}
+
+extern "C" int vasc_global_attn_tokens_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                                           const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                                           const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                           const uint16_t *vt, uint16_t *out, int64_t B, int64_t H, int64_t N,
+                                           int64_t P, int64_t S, int64_t nk, int64_t d,
+                                           const int32_t *block_index, int64_t index_width,
+                                           const int32_t *block_count, float sm_scale, void *stream) {
+  return global_attn_tokens_impl(q_patch, qp_sb, qp_sh, qp_st, q_special, qs_sb, qs_sh, qs_st, k, k_sb, k_sh, k_st,
+                                 vt, out, B, H, N, P, S, nk, d, block_index, index_width, block_count, sm_scale,
+                                 nullptr, 0, stream);
+}
+
+extern "C" int vasc_global_attn_tokens_ws_fwd(const uint16_t *q_patch, int64_t qp_sb, int64_t qp_sh, int64_t qp_st,
+                                              const uint16_t *q_special, int64_t qs_sb, int64_t qs_sh, int64_t qs_st,
+                                              const uint16_t *k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                              const uint16_t *vt, uint16_t *out, int64_t B, int64_t H, int64_t N,
+                                              int64_t P, int64_t S, int64_t nk, int64_t d,
+                                              const int32_t *block_index, int64_t index_width,
+                                              const int32_t *block_count, float sm_scale, void *workspace,
+                                              int64_t workspace_bytes, void *stream) {
+  return global_attn_tokens_impl(q_patch, qp_sb, qp_sh, qp_st, q_special, qs_sb, qs_sh, qs_st, k, k_sb, k_sh, k_st,
+                                 vt, out, B, H, N, P, S, nk, d, block_index, index_width, block_count, sm_scale,
+                                 workspace, workspace_bytes, stream);
 }

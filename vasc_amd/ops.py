@@ -386,6 +386,16 @@ def dense_attn(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, *, scale: flo
     return o
 
 
+def _global_ws(B: int, H: int, n_patch: int, n_special: int, nk: int, width: int, device) -> tuple:
+    """The special queries' split workspace: (tensor or None, pointer, bytes).
+    Fewer than 64 key blocks are never split: not asked for, the call is host time."""
+    if not n_special or nk <= 63 * BLOCK_K:
+        return None, None, 0
+    size = _lib.fn("vasc_global_attn_workspace_size")(B, H, n_patch, n_special, nk, width)
+    ws = torch.empty(size, device=device, dtype=torch.uint8) if size else None
+    return ws, _ptr(ws), size
+
+
 def global_attn(q_patch: torch.Tensor, q_special: torch.Tensor | None, k: torch.Tensor, vt: torch.Tensor,
                 index: torch.Tensor, count: torch.Tensor, *, scale: float | None = None):
     """Patch queries over their listed blocks and special queries over every
@@ -414,9 +424,11 @@ def global_attn(q_patch: torch.Tensor, q_special: torch.Tensor | None, k: torch.
         qs_args = (q_special.data_ptr(), *q_special.stride()[:3])
         os_args = (o_special.data_ptr(), *o_special.stride()[:3])
     scale = D ** -0.5 if scale is None else scale
-    _lib.call("vasc_global_attn_fwd", q_patch.data_ptr(), *q_patch.stride()[:3], *qs_args, k.data_ptr(),
+    ws, ws_ptr, ws_bytes = _global_ws(B, H, n_patch, n_special, nk, index.shape[-1], q_patch.device)
+    _lib.call("vasc_global_attn_ws_fwd", q_patch.data_ptr(), *q_patch.stride()[:3], *qs_args, k.data_ptr(),
               *k.stride()[:3], vt.data_ptr(), o_patch.data_ptr(), *o_patch.stride()[:3], *os_args, B, H, n_patch,
-              n_special, nk, D, index.data_ptr(), index.shape[-1], count.data_ptr(), float(scale), _stream())
+              n_special, nk, D, index.data_ptr(), index.shape[-1], count.data_ptr(), float(scale), ws_ptr, ws_bytes,
+              _stream())
     return o_patch, o_special
 
 
@@ -450,9 +462,10 @@ def global_attn_tokens(q_patch: torch.Tensor, q_special: torch.Tensor | None, k:
         qs_args = (q_special.data_ptr(), *q_special.stride()[:3])
     out = torch.empty(B, N * P, H * D, device=q_patch.device, dtype=torch.bfloat16)
     scale = D ** -0.5 if scale is None else scale
-    _lib.call("vasc_global_attn_tokens_fwd", q_patch.data_ptr(), *q_patch.stride()[:3], *qs_args, k.data_ptr(),
+    ws, ws_ptr, ws_bytes = _global_ws(B, H, n_patch, N * S, nk, index.shape[-1], q_patch.device)
+    _lib.call("vasc_global_attn_tokens_ws_fwd", q_patch.data_ptr(), *q_patch.stride()[:3], *qs_args, k.data_ptr(),
               *k.stride()[:3], vt.data_ptr(), out.data_ptr(), B, H, N, P, S, nk, D, index.data_ptr(),
-              index.shape[-1], count.data_ptr(), float(scale), _stream())
+              index.shape[-1], count.data_ptr(), float(scale), ws_ptr, ws_bytes, _stream())
     return out
 
 
