@@ -31,7 +31,7 @@ struct PackVParams {
 
 // kHalf: V (and K) are IEEE halves, rounded to bf16 as they are read; K only
 // changes its type. One pass over both instead of a cast of each and the pack:
-// 12 frames, 16 heads: 62 -> 21 us.
+// 17 us at 12 frames, 16 heads, where the casts took 25 each and the pack 11.
 template <bool kHalf>
 __global__ __launch_bounds__(256) void pack_v_kernel(const PackVParams p) {
   __shared__ uint16_t tile[kHeadDim][kBlockK + kPad];  // [d][key]
