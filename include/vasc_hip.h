@@ -295,7 +295,9 @@ int vasc_pack_v(const uint16_t *v, int64_t v_sb, int64_t v_sh, int64_t v_st,
  * Replaces _qattn.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf
  * (ZIP:csrc/qattn/attn_cuda.h:19-32) with bf16 inputs instead of int8 +
  * scales. q, o [B,H,nq,d] strided; k [B,H,nk,d] strided; vt from
- * vasc_pack_v. Built variant: d == 64.
+ * vasc_pack_v. o may be q itself (same pointer and strides; the same holds for
+ * the dense and the global entry points); it overlaps no other input. Built
+ * variant: d == 64.
  */
 int vasc_block_sparse_attn_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh,
                                int64_t q_st, const uint16_t *k, int64_t k_sb,

@@ -289,6 +289,52 @@ def test_split_special_queries_match_the_oracle(N, P, S, parts, level):
     assert torch.equal(out[:, :, S:].reshape(1, n_patch, H, 64).transpose(1, 2), op)
 
 
+@pytest.mark.parametrize("kind", ["listed", "dense", "split"])
+@pytest.mark.parametrize("log2_peak", [None, 150.0])
+def test_output_may_lie_on_the_queries(kind, log2_peak):
+    """The attention written over its own queries gives, bit for bit, what it
+    gives beside them, also where the rows' sums leave the range of exponent
+    offset 0 (the first key block's logits near 2^150) and are walked again."""
+    from vasc_amd import _lib, ops
+    H, nq, nk = 2, 300, 4225
+    q, k, v = _rand((1, H, nq, 64), 60), _rand((1, H, nk, 64), 61), _rand((1, H, nk, 64), 62)
+    if log2_peak is not None:  # q0 * k0 / 8 * log2(e)
+        q[..., 0], k[..., 0] = 8.0, 0.0
+        k[:, :, :64, 0] = log2_peak / math.log2(math.e)
+        assert ((q.double() @ k.double().transpose(-1, -2) / 8 * math.log2(math.e)).amax(-1) > 125).all()
+    qc, kc, vt = q.cuda(), k.cuda(), ops.pack_v(v.cuda())
+    qb, nkb = math.ceil(nq / 128), math.ceil(nk / 64)
+    idx = torch.arange(nkb, dtype=torch.int32, device="cuda").expand(1, H, qb, nkb).contiguous()
+    cnt = torch.full((1, H, qb), nkb, dtype=torch.int32, device="cuda")
+    over = qc.clone()
+    if kind == "listed":
+        beside = ops.block_sparse_attn(qc, kc, vt, idx, cnt)
+        ops.block_sparse_attn(over, kc, vt, idx, cnt, out=over)
+    elif kind == "dense":
+        beside = ops.dense_attn(qc, kc, vt)
+        ops.dense_attn(over, kc, vt, out=over)
+    else:  # as the special queries, whose keys are split; one patch query block with one listed block
+        ws_size = _lib.fn("vasc_global_attn_workspace_size")(1, H, 128, nq, nk, 1)
+        assert ws_size > 0
+        qp, op = _rand((1, H, 128, 64), 63).cuda(), torch.empty(1, H, 128, 64, device="cuda", dtype=torch.bfloat16)
+        ws = torch.empty(ws_size, device="cuda", dtype=torch.uint8)
+        first, one = idx[:, :, :1, :1].contiguous(), torch.ones_like(cnt[:, :, :1]).contiguous()
+
+        def special(qs, os_):
+            _lib.call("vasc_global_attn_ws_fwd", qp.data_ptr(), *qp.stride()[:3], qs.data_ptr(), *qs.stride()[:3],
+                      kc.data_ptr(), *kc.stride()[:3], vt.data_ptr(), op.data_ptr(), *op.stride()[:3],
+                      os_.data_ptr(), *os_.stride()[:3], 1, H, 128, nq, nk, 64, first.data_ptr(), 1,
+                      one.data_ptr(), 0.125, ws.data_ptr(), ws_size, torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+        beside = torch.empty_like(qc)
+        special(qc, beside)
+        special(over, over)
+    ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), idx.cpu().numpy(),
+                                    cnt.cpu().numpy())
+    _check(beside, ref)
+    assert torch.equal(over, beside)
+
+
 # ---------------------------------------------------------------- PV post-cut
 def _graded_blocks(nq, nk, levels, seed):
     """Query rows a*e0 (+ small noise) and key block j = levels[j] / c * e0

@@ -33,7 +33,9 @@
 //    Where c is 1 the product goes too. A row sum outside [2^-90, 2^120] (checked after eight
 //    blocks and at the end) sends the workgroup through a second walk with
 //    the running row max as the offset, which also takes blocks outside the
-//    sequence. Checking and rescaling per block cost 2 % of the launch.
+//    sequence. Checking and rescaling per block cost 2 % of the launch. Both
+//    walks take Q from the registers and only the last one stores, so the
+//    output may lie on Q's storage.
 //  * Keys past the sequence end (the partial last block) read the last key's
 //    row: their V rows are zero and the ones operand is zeroed there.
 //  * K and Vt tiles arrive by LDS DMA (global_load_lds_dwordx4) into a
@@ -187,10 +189,9 @@ __device__ __forceinline__ void store_rows(const Params &p, bool sp, int64_t b, 
   }
 }
 
-// The workgroup of bsattn_fwd_kernel again with the running row max as the
-// exponent offset (online softmax), for rows whose sums at offset 0 left the
-// range and for lists that name blocks outside the sequence. Out of line, so
-// that the kernel's registers go to its own loop.
+// The rows of a split special-query workgroup again, every key, with the running
+// row max as the exponent offset (online softmax): combine_kernel's rows whose
+// sums at offset 0 left the range.
 __device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_arg, bool every_block, int wg_arg,
                                            int n_arg) {
   // the arguments arrive in VGPRs: back to scalars, and the parameters through
@@ -458,22 +459,29 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const float c = p.c;
   floatx4 oacc[2][4];  // O^T: [q tile][d tile]
   floatx4 lacc[2];     // row sums of the bf16 probabilities (every register of every lane group alike)
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    lacc[i] = zero4;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
-  }
+  float m[2];          // the second walk's exponent offset of a row (log2 units)
   // operand addresses in the current buffer: row 16 (lr / 8) + lr % 8 of the
   // K tile and row lr of the Vt tile, chunk 4 s + g4
   typedef const __attribute__((address_space(3))) u32x4 *lds_ptr;
-  const int krow = 16 * (lr >> 3) + (lr & 7);
   uint32_t ka_addr[2], va_addr[2];
+  auto start = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    ka_addr[s] = lds0 + krow * 128 + ((4 * s + g4) ^ swz_k(krow)) * 16;
-    va_addr[s] = lds0 + kTile * 2 + lr * 128 + ((4 * s + g4) ^ swz(lr)) * 16;
-  }
+    for (int i = 0; i < 2; ++i) {
+      lacc[i] = zero4;
+      m[i] = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
+    }
+    int lrow = lr;
+    asm volatile("" : "+v"(lrow));  // the addresses are formed again instead of kept for a second walk
+    const int krow = 16 * (lrow >> 3) + (lrow & 7);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      ka_addr[s] = lds0 + krow * 128 + ((4 * s + g4) ^ swz_k(krow)) * 16;
+      va_addr[s] = lds0 + kTile * 2 + lrow * 128 + ((4 * s + g4) ^ swz(lrow)) * 16;
+    }
+  };
+  start();
   auto k_op = [&](int kt, int s) {
     return *reinterpret_cast<lds_ptr>(ka_addr[s] + (32 * (kt >> 1) + 8 * (kt & 1)) * 128);
   };
@@ -538,6 +546,65 @@ void bsattn_fwd_kernel(const AttnParams p) {
     __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, 20, 0);
   };
+  // Probabilities relative to the running row maximum and their products, in
+  // the second walk. lim: the block's keys that exist (more than none).
+  auto compute_online = [&](int lim) __attribute__((always_inline)) {
+    floatx4 S[2][4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4 a = k_op(kt, s);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) S[i][kt] = mfma16(a, qf[i][s], s == 0 ? zero4 : S[i][kt]);
+      }
+    u32x4 pb[2][2];
+    int lane_key = 16 * (g4 >> 1) + 4 * (g4 & 1);
+    asm volatile("" : "+v"(lane_key));  // as in set_ones
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + lane_key + r;
+          S[i][kt][r] = kk < lim ? S[i][kt][r] * c : -INFINITY;
+          mx = fmaxf(mx, S[i][kt][r]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = fmaxf(m[i], mx);
+      const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
+      const float off = mn == -INFINITY ? 0.f : mn;
+      m[i] = mn;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        lacc[i][r] *= alpha;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) oacc[i][t][r] *= alpha;
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(S[i][kt][r] - off),
+                                    __builtin_amdgcn_exp2f(S[i][kt][r + 1] - off));
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) lacc[i] = mfma16(ones, pb[i][s], lacc[i]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const u32x4 a = v_op(t, s);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) oacc[i][t] = mfma16(a, pb[i][s], oacc[i][t]);
+      }
+    }
+  };
   // A row sum out of range, infinite or NaN (bit patterns, so that NaN
   // compares as well).
   auto sums_bad = [&]() __attribute__((always_inline)) {
@@ -555,9 +622,9 @@ void bsattn_fwd_kernel(const AttnParams p) {
   bool out_of_list = false;  // a block outside the sequence was listed
   // The walk: wait for a block's tiles, start the next block's DMA into the
   // other buffer, compute. kIdle: a wave without rows, which only stages its
-  // share of the tiles and keeps the barriers.
-  auto walk = [&](auto idle_wave) __attribute__((always_inline)) {
-    constexpr bool kIdle = decltype(idle_wave)::value;
+  // share of the tiles and keeps the barriers. kOnline: the second walk.
+  auto walk = [&](auto idle_wave, auto online) __attribute__((always_inline)) {
+    constexpr bool kIdle = decltype(idle_wave)::value, kOnline = decltype(online)::value;
     int blk = dense ? blk0 : clist[0];
     int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
     fetch(blk, 0);
@@ -565,7 +632,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma clang loop unroll(disable)
     for (int j = 0; j < nw; ++j) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (j == kCheckAt && __builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
+      if (!kOnline && j == kCheckAt && __builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
       const int lim = valid_keys(blk);
       if (j + 1 < nw) {
         if (dense) {
@@ -578,13 +645,17 @@ void bsattn_fwd_kernel(const AttnParams p) {
         fetch(blk, (j & 1) ^ 1);
       }
       if constexpr (!kIdle) {
-        if (__builtin_expect(lim < kBlockK, 0)) {
-          set_ones(lim);
-          out_of_list |= lim == 0;
+        if constexpr (kOnline) {
+          if (lim > 0) compute_online(lim);
+        } else {
+          if (__builtin_expect(lim < kBlockK, 0)) {
+            set_ones(lim);
+            out_of_list |= lim == 0;
+          }
+          compute();
+          if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
+          if (j == kCheckAt - 1 && sums_bad()) redo = 1;
         }
-        compute();
-        if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
-        if (j == kCheckAt - 1 && sums_bad()) redo = 1;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
           ka_addr[s] ^= kBufBytes;
@@ -595,9 +666,9 @@ void bsattn_fwd_kernel(const AttnParams p) {
   };
   if (n > 0) {
     if (idle) {
-      walk(std::true_type{});
+      walk(std::true_type{}, std::false_type{});
     } else {
-      walk(std::false_type{});
+      walk(std::false_type{}, std::false_type{});
       uint32_t top = 0;  // largest magnitude of O, as bits
 #pragma unroll
       for (int i = 0; i < 2; ++i)
@@ -612,6 +683,21 @@ void bsattn_fwd_kernel(const AttnParams p) {
     }
   }
 
+  __syncthreads();  // every wave is done with the tiles and with redo
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0)) {
+    if (kSplit && sp) {  // combine_kernel walks the rows again
+      if (tid < kBlockQ) p.part[wg * (kBlockQ * (kHeadDim + 1)) + kBlockQ * kHeadDim + tid] = -INFINITY;
+      return;
+    }
+    // again from the first block, with the queries still in registers: nothing
+    // is stored before, so the output may lie on the queries' storage
+    if (idle) {
+      walk(std::true_type{}, std::true_type{});
+    } else {
+      start();
+      walk(std::false_type{}, std::true_type{});
+    }
+  }
   if (kSplit && sp) {
     float *part = p.part + wg * (kBlockQ * (kHeadDim + 1));
 #pragma unroll
@@ -623,16 +709,6 @@ void bsattn_fwd_kernel(const AttnParams p) {
     }
   } else {
     store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
-  }
-  // last, so that no result lives across the call: its stores follow these
-  __syncthreads();  // every wave is done with the tiles and with redo
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0)) {
-    if (kSplit && sp) {  // combine_kernel walks the rows again
-      if (tid < kBlockQ) p.part[wg * (kBlockQ * (kHeadDim + 1)) + kBlockQ * kHeadDim + tid] = -INFINITY;
-      return;
-    }
-    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()), lds0,
-                  kDense, static_cast<int>(unit), n);
   }
 }
 
@@ -661,6 +737,22 @@ void combine_kernel(const AttnParams p) {
         for (int e = 0; e < 4; ++e) acc[c][e] += o[e];
       }
     }
+  }
+  // out of range, marked -inf by a part (weights are never negative), or a sum
+  // of finite parts past the float range
+  bool bad = __float_as_uint(l) - kLowBits > kHighBits - kLowBits;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bad |= (__float_as_uint(acc[c][e]) & 0x7fffffffu) >= 0x7f800000u;
+  bad = bad && qrow < p.nq2;
+  // before the stores, as in bsattn_fwd_kernel
+  if (__syncthreads_or(bad)) {
+    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()),
+                  lds_addr32(tiles), false, static_cast<int>(unit), static_cast<int>(p.nkb));
+    return;
+  }
+  if (qrow < p.nq2) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint16_t *optr = p.o2 + b * p.o2_sb + h * p.o2_sh +
                      (p.tok_p > 0 ? (qrow / p.tok_s) * p.tok_p + qrow % p.tok_s : qrow) * p.o2_st + d0;
@@ -672,18 +764,6 @@ void combine_kernel(const AttnParams p) {
       *reinterpret_cast<u32x4 *>(optr + 4 * c) = v;
     }
   }
-  // out of range, marked -inf by a part (weights are never negative), or a sum
-  // of finite parts past the float range
-  bool bad = __float_as_uint(l) - kLowBits > kHighBits - kLowBits;
-#pragma unroll
-  for (int c = 0; c < 8; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bad |= (__float_as_uint(acc[c][e]) & 0x7fffffffu) >= 0x7f800000u;
-  bad = bad && qrow < p.nq2;
-  __syncthreads();  // these stores come before those of the second walk
-  if (__syncthreads_or(bad))
-    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()),
-                  lds_addr32(tiles), false, static_cast<int>(unit), static_cast<int>(p.nkb));
 }
 
 // The PV post-cut (qk_int_sv_f16_cuda_sm80.cuh:291-381): 4 waves x 32 query
