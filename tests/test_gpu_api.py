@@ -434,6 +434,47 @@ def test_global_layer_forward_dense_limit():
     assert err.max() < 6e-2 and err.mean() < 6e-3, (err.max().item(), err.mean().item())
 
 
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("std", [1.0, 2.0])
+def test_layers_without_norms_round_the_queries_once(rope, std):
+    """At sparsity 0, a layer with identity norms gives, bit for bit, the dense
+    attention of the queries as the layout packs them: bf16 from the projection
+    (special tokens, and every token without a rope) or rounded once after the
+    rotation. No copy with the softmax scale in it is rounded on the way."""
+    from types import SimpleNamespace
+
+    from vasc_amd import ops
+    from vasc_amd.aggregator import RotaryPositionEmbedding2D
+    from vasc_amd.attention import adaptive_sparse_attention_forward
+    N, Hp, Wp, S, heads, dim = 2, 10, 13, 5, 4, 256
+    P = Hp * Wp + S
+    table = RotaryPositionEmbedding2D() if rope else None
+    qkv = (torch.randn(1, N * P, 3 * dim, generator=torch.Generator().manual_seed(8)) * std).to(torch.bfloat16).cuda()
+    m = SimpleNamespace(qkv=lambda x: qkv, proj=torch.nn.Identity(), q_norm=torch.nn.Identity(),
+                        k_norm=torch.nn.Identity(), rope=table)
+    ys, xs = torch.meshgrid(torch.arange(Hp), torch.arange(Wp), indexing="ij")
+    patch_pos = torch.stack([ys.reshape(-1), xs.reshape(-1)], -1) + 1
+    pos = torch.cat([torch.zeros(S, 2, dtype=torch.long), patch_pos]).repeat(N, 1).unsqueeze(0).cuda()
+    x = torch.zeros(1, N * P, dim, device="cuda", dtype=torch.bfloat16)
+    saved = {k: os.environ.pop(k) for k in list(os.environ) if k.startswith("SPARSE_VGGT_")}
+    try:
+        os.environ["SPARSE_VGGT_OFFICIAL_MASK"] = "1"
+        out = adaptive_sparse_attention_forward(m, x, pos, sparse_ratio=0.0, num_special_tokens=S, num_heads=heads,
+                                                routing_state={})
+    finally:
+        os.environ.pop("SPARSE_VGGT_OFFICIAL_MASK", None)
+        os.environ.update(saved)
+    q, k, v = qkv.view(1, N * P, 3, heads, 64).unbind(2)
+    qp, qs, kp, vp = ops.pack_qkv(q, k, v, N, P, S, pos=pos if rope else None,
+                                  rope_tables=table.tables(64, x.device) if rope else None)
+    special = q.view(1, N, P, heads, 64)[:, :, :S].reshape(1, N * S, heads, 64).transpose(1, 2)
+    assert torch.equal(qs, special)  # position 0 does not rotate
+    vt = ops.pack_v(vp)
+    ref = torch.cat([ops.dense_attn(qs, kp, vt).unflatten(2, (N, S)),
+                     ops.dense_attn(qp, kp, vt).unflatten(2, (N, P - S))], dim=3)
+    assert torch.equal(out, ref.permute(0, 2, 3, 1, 4).reshape(1, N * P, dim))
+
+
 def _check_stats(got, ref, where):
     assert set(got) >= set(ref), (where, sorted(set(ref) - set(got)))
     for key, val in ref.items():

@@ -124,11 +124,15 @@ def adaptive_sparse_attention_forward(self, x: torch.Tensor, pos: torch.Tensor, 
     if pool_mode == "avg" and n_patch > 0 and fused_layout_supported(self):
         # layout, V tiles, block means and value innovation in one pass
         tables = rope.tables(hd, x.device) if rope is not None else None
-        # the softmax scale goes into the queries before their one rounding to bf16
+        q_norm = layer_norm_args(self.q_norm)
+        # the softmax scale goes into normed queries before their one rounding to bf16; without a norm the special
+        # tokens (and without a rope all) are bf16 as they come, and a scaled copy would be a rounding more:
+        # 2.3e-3 -> 2.8e-3 from float64 at unit scale, 2.2e-3 -> 3.8e-3 at twice that
+        q_scale, scale = (1.0, None) if q_norm is None else (ops.LOG2E / math.sqrt(hd), ops.LN2)
         q_patch, q_special, k_re, vt, pq, pk, innovation, _ = ops.pack_global(
-            qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], N, P, S, q_norm=layer_norm_args(self.q_norm),
+            qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], N, P, S, q_norm=q_norm,
             k_norm=layer_norm_args(self.k_norm), pos=pos if rope is not None else None, rope_tables=tables,
-            innovation=vasc_mode, q_scale=ops.LOG2E / math.sqrt(hd))
+            innovation=vasc_mode, q_scale=q_scale)
         # the ledger's QK-order priority (the cleaned score) from the same launch
         attn_pooled, priority = ops.pooled_softmax(pq, pk, scale=1.0 / math.sqrt(hd), priority=True) \
             if vasc_mode else (ops.pooled_softmax(pq, pk, scale=1.0 / math.sqrt(hd)), None)
@@ -136,7 +140,7 @@ def adaptive_sparse_attention_forward(self, x: torch.Tensor, pos: torch.Tensor, 
             q_patch, q_special, k_re, None, attn_pooled, sparse_ratio=sparse_ratio, cdf_threshold=cdf_threshold,
             layer_idx=layer_idx, routing_state=routing_state, num_patch_tokens=n_patch,
             want_sparsity=aux_output_store is not None, _innovation=innovation, token_layout=(N, P, S), _vt=vt,
-            _priority=priority, _scale=ops.LN2, _cfg=cfg, **research)
+            _priority=priority, _scale=scale, _cfg=cfg, **research)
         return _finish(self, x, tokens_out, sparsity, aux_output_store)
     if fused_layout_supported(self):
         tables = rope.tables(hd, x.device) if rope is not None else None
