@@ -289,6 +289,32 @@ def test_split_special_queries_match_the_oracle(N, P, S, parts, level):
     assert torch.equal(out[:, :, S:].reshape(1, n_patch, H, 64).transpose(1, 2), op)
 
 
+@pytest.mark.parametrize("split", [False, True])
+def test_differences_of_huge_logits_are_not_rounded_away(split):
+    """Logits of 2^20 whose differences of 0, 1 and 2 decide the weights: every
+    score is a whole number below 2^24, exact in float32, while its product with
+    log2(e) / 8 alone would be rounded to a multiple of 1/8 (4 percent of a weight)."""
+    from vasc_amd import ops
+    H, nk, nq = 1, 4225, 130
+    q, k, v = torch.zeros(1, H, nq, 64), torch.zeros(1, H, nk, 64), _rand((1, H, nk, 64), 65)
+    q[..., 0], q[..., 1] = 2048.0, 1.0
+    k[..., 0] = 4096.0
+    k[..., 1] = -8.0 * (torch.arange(nk) % 3)
+    k[:, :, 12:, 1] -= 4096.0  # twelve keys carry the weight
+    q, k = q.to(torch.bfloat16), k.to(torch.bfloat16)
+    nkb, qb = math.ceil(nk / 64), math.ceil(nq / 128)
+    full = torch.arange(nkb, dtype=torch.int32).expand(1, H, qb, nkb).contiguous()
+    cnt = torch.full((1, H, qb), nkb, dtype=torch.int32)
+    ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), full.numpy(), cnt.numpy())
+    qc, kc, vt = q.cuda(), k.cuda(), ops.pack_v(v.cuda())
+    if split:  # as special queries, beside one patch query block with one listed block
+        _check(ops.global_attn(qc[:, :, :128], qc, kc, vt, full[:, :, :1, :1].cuda(), torch.ones_like(cnt[:, :, :1]).cuda())[1],
+               ref)
+    else:
+        _check(ops.block_sparse_attn(qc, kc, vt, full.cuda(), cnt.cuda()), ref)
+        _check(ops.dense_attn(qc, kc, vt), ref)
+
+
 @pytest.mark.parametrize("kind", ["listed", "dense", "split"])
 @pytest.mark.parametrize("log2_peak", [None, 150.0])
 def test_output_may_lie_on_the_queries(kind, log2_peak):

@@ -295,12 +295,12 @@ __device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_a
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + 16 * (g4 >> 1) + 4 * (g4 & 1) + r;
-          S[i][kt][r] = kk < lim ? S[i][kt][r] * p.c : -INFINITY;
+          S[i][kt][r] = kk < lim ? S[i][kt][r] : -INFINITY;
           mx = fmaxf(mx, S[i][kt][r]);
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[i], mx);
+      const float mn = fmaxf(m[i], mx * p.c);
       const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
       const float off = mn == -INFINITY ? 0.f : mn;
       m[i] = mn;
@@ -315,8 +315,8 @@ __device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_a
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
-          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(S[i][kt][r] - off),
-                                    __builtin_amdgcn_exp2f(S[i][kt][r + 1] - off));
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(S[i][kt][r], p.c, -off)),
+                                    __builtin_amdgcn_exp2f(fmaf(S[i][kt][r + 1], p.c, -off)));
         }
     }
 #pragma unroll
@@ -569,12 +569,12 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + lane_key + r;
-          S[i][kt][r] = kk < lim ? S[i][kt][r] * c : -INFINITY;
+          S[i][kt][r] = kk < lim ? S[i][kt][r] : -INFINITY;
           mx = fmaxf(mx, S[i][kt][r]);
         }
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[i], mx);
+      const float mn = fmaxf(m[i], mx * c);
       const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
       const float off = mn == -INFINITY ? 0.f : mn;
       m[i] = mn;
@@ -589,8 +589,9 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
-          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(S[i][kt][r] - off),
-                                    __builtin_amdgcn_exp2f(S[i][kt][r + 1] - off));
+          // one rounding of c S - m, not one of c S before it
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(S[i][kt][r], c, -off)),
+                                    __builtin_amdgcn_exp2f(fmaf(S[i][kt][r + 1], c, -off)));
         }
     }
 #pragma unroll
