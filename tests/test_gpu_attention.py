@@ -154,10 +154,10 @@ def test_c1_layer_topk_lists():
 
 @pytest.mark.parametrize("case", ["high", "low", "mixed"])
 def test_extreme_logits_take_the_exact_path(case):
-    """Logits far outside the fast path's range: above 64 in log2 units (the
-    block sum overflows 2^64) or all below -126 (every probability would
-    underflow). The kernel must move its exponent offset and still match the
-    float64 softmax."""
+    """Logits far outside the fast path's range: row sums above 2^120 (the
+    largest of them above 2^130) or all logits below -126 in log2 units (every
+    probability would underflow). The kernel must move its exponent offset and
+    still match the float64 softmax."""
     from vasc_amd import ops
     B, H, nq, nk, D = 1, 2, 256, 640, 64
     g = torch.Generator().manual_seed(21)
@@ -167,8 +167,8 @@ def test_extreme_logits_take_the_exact_path(case):
     u = torch.randn(D, generator=g)
     u = u / u.norm() * 8.0
     if case == "high":
-        # logit std ~ 0.18 * 4 * 4 * 8 = 23: row maxima 50..105
-        q, k = q * 4.0, k * 4.0
+        # log2 logit std ~ 0.18 * 6 * 6 * 8 = 52: row maxima 100..220
+        q, k = q * 6.0, k * 6.0
     else:
         # every key ~ -4u: rows ~ +4u sit near -185 (all below -126), rows
         # ~ -4u near +185; "mixed" interleaves those with ordinary rows
@@ -183,6 +183,8 @@ def test_extreme_logits_take_the_exact_path(case):
     q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
     qb, nkb = math.ceil(nq / 128), math.ceil(nk / 64)
     idx, cnt = _lists(B, H, qb, nkb, 22, density=0.6)
+    sums = _log2_sums(q, k, idx, cnt)
+    assert {"high": sums.max() > 130, "low": sums.max() < -100, "mixed": sums.max() > 130 and sums.min() < -100}[case]
     out = ops.block_sparse_attn(q.cuda(), k.cuda(), ops.pack_v(v.cuda()), torch.from_numpy(idx).cuda(),
                                 torch.from_numpy(cnt).cuda())
     ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), idx, cnt)
@@ -192,28 +194,45 @@ def test_extreme_logits_take_the_exact_path(case):
     _check(dense, OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), *dl))
 
 
-@pytest.mark.parametrize("hot", [0.0, 30.0])
-@pytest.mark.parametrize("nblk,at,reverse", [(1, 0, False), (7, 6, False), (8, 7, True), (9, 8, False), (9, 0, True),
-                                             (20, 7, False), (20, 8, True), (20, 19, False)])
+def _log2_sums(q, k, idx, cnt):
+    """Row sums of the listed keys' exponentials, log2, in float64."""
+    s = q.double() @ k.double().transpose(-1, -2).contiguous() * (q.shape[-1] ** -0.5 * math.log2(math.e))
+    keep = torch.zeros(*idx.shape[:3], math.ceil(k.shape[2] / 64), dtype=torch.bool)
+    for at in np.ndindex(*cnt.shape):
+        keep[at][torch.from_numpy(idx[at][:cnt[at]]).long()] = True
+    keep = keep.repeat_interleave(64, -1)[..., :k.shape[2]].repeat_interleave(128, 2)[:, :, :q.shape[2]]
+    return torch.logsumexp(s.masked_fill(~keep, -math.inf) * math.log(2), -1) / math.log(2)
+
+
+@pytest.mark.parametrize("hot", [None, "peak", "ramp", "low"])
+@pytest.mark.parametrize("nblk,at,reverse", [(1, 0, False), (2, 1, False), (7, 6, False), (8, 7, True), (9, 8, False),
+                                             (9, 0, True), (10, 9, False), (20, 7, False), (20, 8, True), (20, 9, False),
+                                             (20, 19, False), (27, 24, False), (27, 25, True), (60, 56, False),
+                                             (60, 57, False)])
 def test_range_exit_at_every_point_of_the_walk(nblk, at, reverse, hot):
-    """Block ``at`` lifts every third row's logits by about ``hot`` * 8 * log2 e
-    (above the range of exponent offset 0; hot = 0 stays inside it), before and
-    after the kernel's early look at its row sums, in lists of either order that
-    hold the partial last block, with waves that own no rows (nq = 130). Same
+    """Rows whose sums leave the range of exponent offset 0, before, at and after
+    the points where the kernel looks at them (after blocks 0, 8, 24, 56 and the
+    last), in lists of either order that hold the partial last block, with waves
+    that own no rows (nq = 130). Every third row is out: "peak": block ``at`` near
+    2^180; "ramp": each block 2^70 above the one before, so that the second walk
+    moves its offset in every block; "low": every logit near 2^-180. Same
     tolerance as the other extreme-logit cases: bf16 probabilities of a float64
     softmax."""
     from vasc_amd import ops
     B, H, nq, nk, D = 1, 2, 130, 64 * nblk - 31, 64
-    q, k, v = (_rand((B, H, n, D), 30 + i).float() for i, n in enumerate((nq, nk, nk)))
-    u = torch.zeros(D)
-    u[:16] = 4.0 ** 0.5 / 2
-    if hot:
-        q[:, :, ::3] += hot / 4 * u
-        k[:, :, 64 * at:64 * at + 64] += 4.0 * u
-    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    q, k, v = (_rand((B, H, n, D), 30 + i) for i, n in enumerate((nq, nk, nk)))
+    q[..., 0] = 0.0
     order = np.arange(nblk)[::-1] if reverse else np.arange(nblk)
     idx = np.ascontiguousarray(np.broadcast_to(order.astype(np.int32), (B, H, 2, nblk)))
     cnt = np.full((B, H, 2), nblk, np.int32)
+    if hot:
+        q[:, :, ::3, 0] = 8.0  # log2 logit: q0 * k0 / 8 * log2(e)
+        level = {"peak": torch.where(torch.arange(nblk) == at, 180.0, 0.0), "ramp": 70.0 * (torch.arange(nblk) + 2),
+                 "low": torch.full((nblk,), -180.0)}[hot]
+        k[..., 0] = (level / math.log2(math.e)).to(torch.bfloat16).repeat_interleave(64)[:nk]
+        sums = _log2_sums(q, k, idx, cnt)
+        assert ((sums[:, :, ::3] < -150) if hot == "low" else (sums[:, :, ::3] > 125)).all()
+        assert (sums[:, :, 1::3].abs() < 30).all()
     qc, kc, vt = q.cuda(), k.cuda(), ops.pack_v(v.cuda())
     out = ops.block_sparse_attn(qc, kc, vt, torch.from_numpy(idx).cuda(), torch.from_numpy(cnt).cuda())
     ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), idx, cnt)

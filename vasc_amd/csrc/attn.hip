@@ -30,12 +30,15 @@
 //  * Softmax is invariant to the exponent offset, which only has to keep the
 //    probabilities inside fp32/bf16 range. The walk uses offset 0:
 //    P = exp2(c S) on the exact fp32 logits, no max, no rescale, no branch.
-//    Where c is 1 the product goes too. A row sum outside [2^-90, 2^120] (checked after eight
-//    blocks and at the end) sends the workgroup through a second walk with
-//    the running row max as the offset, which also takes blocks outside the
-//    sequence. Checking and rescaling per block cost 2 % of the launch. Both
-//    walks take Q from the registers and only the last one stores, so the
-//    output may lie on Q's storage.
+//    Where c is 1 the product goes too. A row sum outside [2^-60, 2^120]
+//    (looked at after blocks 0, 8, 24, 56, .. and at the end) sends the
+//    workgroup through a second walk, whose offset follows the row maximum and
+//    which also takes blocks outside the sequence. Checking and rescaling per
+//    block cost 2 % of the launch. Both walks take Q from the registers and
+//    only the last one stores, so the output may lie on Q's storage. Over 33312
+//    keys, 16 heads, 132 blocks a row, q and k of std 1 / 4 / 8 take 1.06 /
+//    1.15 / 1.11 ms (offset moved per block in the first walk: 1.16 / 1.19 /
+//    1.58; second walk with a new maximum each block: 1.06 / 1.88 / 1.48).
 //  * Keys past the sequence end (the partial last block) read the last key's
 //    row: their V rows are zero and the ones operand is zeroed there.
 //  * K and Vt tiles arrive by LDS DMA (global_load_lds_dwordx4) into a
@@ -131,11 +134,16 @@ __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 // below m that they lose precision).
 constexpr float kHigh = 18446744073709551616.0f;  // 2^64
 constexpr float kLow = 8.673617379884035e-19f;    // 2^-60
-// Row sums at exponent offset 0 are good in [2^-90, 2^120]: below, flushed
-// probabilities (under 2^-126) could add up to more than 2^-23 of the sum;
-// above, the largest ones near overflow. The accumulated outputs are checked
-// for finiteness beside them.
-constexpr uint32_t kHighBits = 0x7b800000u, kLowBits = 0x12800000u;
+// Row sums at exponent offset 0 are good in [2^-60, 2^120]: below, products of
+// small probabilities and small values would be flushed; above, the largest
+// ones near overflow. The accumulated outputs are checked for finiteness beside
+// them. A walk whose sums will leave the range is better left early: above 2^72
+// after the first block (3.9 standard deviations, the largest of its 8192
+// scores, where the walk's largest of a million lie at 4.9 to 5.2), later above
+// 2^104. A needless second walk costs 5 to 10 %, a late one twice the time.
+constexpr uint32_t kHighBits = 0x7b800000u, kLaterBits = 0x73800000u, kFirstBits = 0x63800000u, kLowBits = 0x21800000u;
+// Second walk (see compute_online).
+constexpr float kRaise = 64.f, kMargin = 32.f;
 
 // LDS DMA without a memory clobber (the waits and barriers that order it are
 // explicit); uniform list reads then stay on the scalar unit.
@@ -155,7 +163,6 @@ __device__ __forceinline__ floatx4 mfma16(u32x4 a, u32x4 b, floatx4 c) {
 // LDS chunk swizzle of K tile row r in bsattn_fwd_kernel (see above).
 __device__ __forceinline__ int swz_k(int r) { return ((r >> 1) & 3) | ((r >> 2) & 4); }
 
-constexpr int kCheckAt = 8;  // blocks walked before the first look at the row sums
 
 typedef const __attribute__((address_space(4))) AttnParams ConstParams;
 
@@ -459,7 +466,8 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const float c = p.c;
   floatx4 oacc[2][4];  // O^T: [q tile][d tile]
   floatx4 lacc[2];     // row sums of the bf16 probabilities (every register of every lane group alike)
-  float m[2];          // the second walk's exponent offset of a row (log2 units)
+  float m[2];          // second walk: the row's exponent offset
+  bool unset = true;   // second walk: no block has set the offset
   // operand addresses in the current buffer: row 16 (lr / 8) + lr % 8 of the
   // K tile and row lr of the Vt tile, chunk 4 s + g4
   typedef const __attribute__((address_space(3))) u32x4 *lds_ptr;
@@ -468,7 +476,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       lacc[i] = zero4;
-      m[i] = -INFINITY;
+      m[i] = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
     }
@@ -546,8 +554,11 @@ void bsattn_fwd_kernel(const AttnParams p) {
     __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, 20, 0);
   };
-  // Probabilities relative to the running row maximum and their products, in
-  // the second walk. lim: the block's keys that exist (more than none).
+  // The second walk's block: probabilities relative to the row's offset m, which
+  // follows the row maximum in steps: it moves where a score passes it by kRaise,
+  // to kMargin above the block's maximum, so that few blocks move it (the first
+  // block that has keys sets it). A whole number, so that the sums' rescaling is
+  // exact. lim: the block's keys that exist (more than none).
   auto compute_online = [&](int lim) __attribute__((always_inline)) {
     floatx4 S[2][4];
 #pragma unroll
@@ -558,42 +569,57 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) S[i][kt] = mfma16(a, qf[i][s], s == 0 ? zero4 : S[i][kt]);
       }
-    u32x4 pb[2][2];
-    int lane_key = 16 * (g4 >> 1) + 4 * (g4 & 1);
-    asm volatile("" : "+v"(lane_key));  // as in set_ones
+    if (__builtin_expect(lim < kBlockK, 0)) {
+      int lane_key = 16 * (g4 >> 1) + 4 * (g4 & 1);
+      asm volatile("" : "+v"(lane_key));  // as in set_ones
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            S[i][kt][r] = 32 * (kt >> 1) + 8 * (kt & 1) + lane_key + r < lim ? S[i][kt][r] : -INFINITY;
+    }
+    float mx[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      float mx = -INFINITY;
+      mx[i] = S[i][0][0];
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
+        for (int r = 0; r < 4; ++r) mx[i] = fmaxf(mx[i], S[i][kt][r]);
+    }
+    const float over = fmaxf(fmaf(mx[0], c, -m[0]), fmaf(mx[1], c, -m[1]));
+    if (__builtin_expect(unset || __ballot(over > kRaise) != 0, 0)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float top = fmaxf(mx[i], __shfl_xor(mx[i], 16));
+        top = fmaxf(top, __shfl_xor(top, 32)) * c;
+        float to = __builtin_rintf(top + kMargin);
+        if ((!unset && top <= m[i]) || (__float_as_uint(top) & 0x7f800000u) == 0x7f800000u) to = m[i];
+        const float alpha = unset ? 0.f : __builtin_amdgcn_exp2f(m[i] - to);
+        m[i] = to;
+#pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + lane_key + r;
-          S[i][kt][r] = kk < lim ? S[i][kt][r] : -INFINITY;
-          mx = fmaxf(mx, S[i][kt][r]);
+          lacc[i][r] *= alpha;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) oacc[i][t][r] *= alpha;
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[i], mx * c);
-      const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
-      const float off = mn == -INFINITY ? 0.f : mn;
-      m[i] = mn;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lacc[i][r] *= alpha;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) oacc[i][t][r] *= alpha;
       }
+      unset = false;
+    }
+    u32x4 pb[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
           // one rounding of c S - m, not one of c S before it
-          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(S[i][kt][r], c, -off)),
-                                    __builtin_amdgcn_exp2f(fmaf(S[i][kt][r + 1], c, -off)));
+          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(S[i][kt][r], c, -m[i])),
+                                    __builtin_amdgcn_exp2f(fmaf(S[i][kt][r + 1], c, -m[i])));
         }
-    }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -608,10 +634,10 @@ void bsattn_fwd_kernel(const AttnParams p) {
   };
   // A row sum out of range, infinite or NaN (bit patterns, so that NaN
   // compares as well).
-  auto sums_bad = [&]() __attribute__((always_inline)) {
+  auto sums_bad = [&](uint32_t high) __attribute__((always_inline)) {
     bool x = false;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) x |= __float_as_uint(lacc[i][0]) - kLowBits > kHighBits - kLowBits;
+    for (int i = 0; i < 2; ++i) x |= __float_as_uint(lacc[i][0]) - kLowBits > high - kLowBits;
     return __ballot(x) != 0;
   };
 
@@ -629,11 +655,14 @@ void bsattn_fwd_kernel(const AttnParams p) {
     int blk = dense ? blk0 : clist[0];
     int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
     fetch(blk, 0);
-    int nw = n;
+    int nw = n, look = 0;  // look: the block after which the row sums are looked at next (0, 8, 24, 56, ..)
 #pragma clang loop unroll(disable)
     for (int j = 0; j < nw; ++j) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (!kOnline && j == kCheckAt && __builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
+      if (!kOnline && j == look + 1) {
+        if (__builtin_amdgcn_readfirstlane(redo)) nw = 0;
+        look = 2 * look + 8;
+      }
       const int lim = valid_keys(blk);
       if (j + 1 < nw) {
         if (dense) {
@@ -653,9 +682,9 @@ void bsattn_fwd_kernel(const AttnParams p) {
             set_ones(lim);
             out_of_list |= lim == 0;
           }
-          compute();
+          if (nw) compute();
           if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
-          if (j == kCheckAt - 1 && sums_bad()) redo = 1;
+          if (j == look && sums_bad(look ? kLaterBits : kFirstBits)) redo = 1;
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -680,7 +709,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
             const uint32_t o = __float_as_uint(oacc[i][t][r]) & 0x7fffffffu;
             top = o > top ? o : top;
           }
-      if (sums_bad() || __ballot(top >= 0x7f800000u) != 0 || out_of_list) redo = 1;
+      if (sums_bad(kHighBits) || __ballot(top >= 0x7f800000u) != 0 || out_of_list) redo = 1;
     }
   }
 
