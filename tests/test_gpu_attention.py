@@ -242,9 +242,10 @@ def test_range_exit_at_every_point_of_the_walk(nblk, at, reverse, hot):
 
 @pytest.mark.parametrize("N,P,S,H", [(1, 129, 1, 1), (3, 47, 5, 3), (2, 130, 0, 9)])
 def test_prescaled_queries_match_the_oracle(N, P, S, H):
-    """Queries packed with the softmax scale (one bf16 rounding of q * scale
-    instead of one of q): the layout differs in q only, the pooled means not at
-    all, and the prescaled attention stays within the file's tolerance of the float64 softmax of the unscaled float32 queries."""
+    """Queries packed with the softmax scale: the layout differs in q only, the
+    pooled means not at all, and the attention of patch and special queries stays
+    within the file's tolerance of the float64 softmax of the unscaled queries
+    (which have no norm here, so that the scaled copy is a rounding more)."""
     from vasc_amd import ops
     T = N * P
     qkv = _rand((1, T, 3, H, 64), 40).cuda()
@@ -268,6 +269,13 @@ def test_prescaled_queries_match_the_oracle(N, P, S, H):
                                  scale=ops.LN2)
     patch = out.view(1, N, P, H, 64)[:, :, S:].reshape(1, np_, H, 64).transpose(1, 2)
     _check(patch, rows)
+    if S:
+        n_sp = N * S
+        full = np.broadcast_to(np.arange(nkb, dtype=np.int32), (1, H, math.ceil(n_sp / 128), nkb))
+        _check(out.view(1, N, P, H, 64)[:, :, :S].reshape(1, n_sp, H, 64).transpose(1, 2),
+               OA.block_sparse_attention(ref[1].float().cpu().numpy(), ko.float().cpu().numpy(),
+                                         ops.pack_qkv(q, k, v, N, P, S)[3].float().cpu().numpy(), full,
+                                         np.full(full.shape[:3], nkb)))
 
 
 @pytest.mark.parametrize("level", [None, "high", "low"])
@@ -306,6 +314,52 @@ def test_split_special_queries_match_the_oracle(N, P, S, parts, level):
     out = ops.global_attn_tokens(qp, qs, kc, vt, idx.cuda(), cnt.cuda(), N, P, S).view(1, N, P, H, 64)
     assert torch.equal(out[:, :, :S].reshape(1, n_sp, H, 64).transpose(1, 2), os_)
     assert torch.equal(out[:, :, S:].reshape(1, n_patch, H, 64).transpose(1, 2), op)
+
+
+@pytest.mark.parametrize("unit", [False, True])
+@pytest.mark.parametrize("level", [None, "high", "low", "parts"])
+def test_split_special_queries_in_batches(level, unit):
+    """The key split with two batch entries, strided queries and both forms of
+    the kernel (the plain scale; queries that hold the scale, sm_scale = ln 2).
+    "high" and "low" as above; "parts": the last two of three parts near 2^180 with
+    comparable weights, the first at 2^0, so that parts of different offsets meet
+    in the combination."""
+    from vasc_amd import _lib, ops
+    B, H, N, P, S = 2, 2, 2, 3201, 3
+    nk, n_patch, n_sp = N * P, N * (P - S), N * S
+    nkb, qb, parts = math.ceil(nk / 64), math.ceil(n_patch / 128), 3
+    k, v = _rand((B, nk, H, 64), 71), _rand((B, H, nk, 64), 72)
+    q = _rand((B, nk, H, 64), 70)
+    if level is not None:
+        q[..., 0] = 8.0
+        k[..., 0] = 0.0
+        if level == "high":
+            k[:, :64, :, 0] = 150.0 / math.log2(math.e)
+        elif level == "low":
+            k[..., 0] = -160.0 / math.log2(math.e)
+        else:
+            k[:, math.ceil(nkb / parts) * 64:, :, 0] = 180.0 / math.log2(math.e)
+    scale = None
+    if unit:
+        q, scale = (q.float() * (ops.LOG2E / 8)).to(torch.bfloat16), ops.LN2
+    q, k = q.cuda().transpose(1, 2), k.cuda().transpose(1, 2)
+    qp, qs, vt = q[:, :, :n_patch], q[:, :, n_patch:], ops.pack_v(v.cuda())
+    W = 40  # lists of 40 blocks: 100 key blocks in parts of at least 32 blocks, about as long as the lists
+    idx = (torch.arange(W, dtype=torch.int32) * 2 + 1).expand(B, H, qb, W).contiguous()
+    cnt = torch.full((B, H, qb), W, dtype=torch.int32)
+    size = _lib.fn("vasc_global_attn_workspace_size")(B, H, n_patch, n_sp, nk, W)
+    assert size == B * H * math.ceil(n_sp / 128) * parts * 128 * 65 * 4
+    op, os_ = ops.global_attn(qp, qs, k, vt, idx.cuda(), cnt.cuda(), scale=scale)
+    out = ops.global_attn_tokens(qp, qs, k, vt, idx.cuda(), cnt.cuda(), N, P, S, scale=scale).view(B, N, P, H, 64)
+    assert torch.equal(out[:, :, :S].reshape(B, n_sp, H, 64).transpose(1, 2), os_)
+    assert torch.equal(out[:, :, S:].reshape(B, n_patch, H, 64).transpose(1, 2), op)
+    kn, vn = k.cpu().float().numpy(), v.float().numpy()
+    full = np.broadcast_to(np.arange(nkb, dtype=np.int32), (B, H, 1, nkb))
+    _check(os_, OA.block_sparse_attention(qs.cpu().float().numpy(), kn, vn, full, np.full((B, H, 1), nkb), scale=scale))
+    some = [0, qb - 1]
+    ref = OA.block_sparse_attention(qp.cpu().float().numpy(), kn, vn, idx.numpy(), cnt.numpy(), scale=scale, q_blocks=some)
+    for i in some:
+        _check(op[:, :, 128 * i:128 * i + 128], ref[:, :, 128 * i:128 * i + 128])
 
 
 @pytest.mark.parametrize("split", [False, True])

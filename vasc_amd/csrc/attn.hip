@@ -110,7 +110,7 @@ struct AttnParams {
   int64_t pv_w;
   // key split of the special queries: nsplit workgroups walk split_blocks key
   // blocks each and leave float32 partial results, [num_wg2][nsplit][128 rows]
-  // of 64 sums of P V, then of the row sums
+  // of 64 outputs of the part's keys alone, then of log2 of the row sums
   int32_t nsplit, split_blocks;
   float *part;
 };
@@ -145,6 +145,8 @@ constexpr uint32_t kHighBits = 0x7b800000u, kLaterBits = 0x73800000u, kFirstBits
 // Second walk (see compute_online).
 constexpr float kRaise = 64.f, kMargin = 32.f;
 
+constexpr int kMaxSplit = 8;  // workgroups that share a special-query block's keys
+
 // LDS DMA without a memory clobber (the waits and barriers that order it are
 // explicit); uniform list reads then stay on the scalar unit.
 __device__ __forceinline__ void dma16(const void *sbase, uint32_t voff_bytes, uint32_t lds_addr) {
@@ -164,12 +166,9 @@ __device__ __forceinline__ floatx4 mfma16(u32x4 a, u32x4 b, floatx4 c) {
 __device__ __forceinline__ int swz_k(int r) { return ((r >> 1) & 3) | ((r >> 2) & 4); }
 
 
-typedef const __attribute__((address_space(4))) AttnParams ConstParams;
-
 // Normalised results of a wave's two query tiles; a row without any
 // probability is zero. sp: the special-query outputs.
-template <typename Params>
-__device__ __forceinline__ void store_rows(const Params &p, bool sp, int64_t b, int64_t h, int64_t row0, int64_t nq,
+__device__ __forceinline__ void store_rows(const AttnParams &p, bool sp, int64_t b, int64_t h, int64_t row0, int64_t nq,
                                            int lr, int g4, const floatx4 (&oacc)[2][4], const floatx4 (&lacc)[2]) {
   uint16_t *odst = sp ? p.o2 + b * p.o2_sb + h * p.o2_sh : p.o + b * p.o_sb + h * p.o_sh;
   const int64_t o_st = sp ? p.o2_st : p.o_st;
@@ -194,152 +193,6 @@ __device__ __forceinline__ void store_rows(const Params &p, bool sp, int64_t b, 
       *reinterpret_cast<uint2 *>(optr + 16 * t + 4 * g4) = v;
     }
   }
-}
-
-// The rows of a split special-query workgroup again, every key, with the running
-// row max as the exponent offset (online softmax): combine_kernel's rows whose
-// sums at offset 0 left the range.
-__device__ __noinline__ void bsattn_online(const AttnParams *pp, uint32_t lds0_arg, bool every_block, int wg_arg,
-                                           int n_arg) {
-  // the arguments arrive in VGPRs: back to scalars, and the parameters through
-  // the constant address space
-  auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); };
-  const uint64_t pa = reinterpret_cast<uint64_t>(pp);
-  const ConstParams &p = *reinterpret_cast<const ConstParams *>(
-      (static_cast<uint64_t>(uniform(static_cast<uint32_t>(pa >> 32))) << 32) | uniform(static_cast<uint32_t>(pa)));
-  const uint32_t lds0 = uniform(lds0_arg);
-  const int wg = static_cast<int>(uniform(static_cast<uint32_t>(wg_arg)));
-  const int n = static_cast<int>(uniform(static_cast<uint32_t>(n_arg)));
-  const bool dense = every_block || static_cast<int64_t>(blockIdx.x) < p.num_wg2_slots;
-  const bool sp = dense && !every_block;
-  const int64_t nqb = sp ? p.nq2b : p.nqb;
-  const int qb = static_cast<int>(wg % nqb);
-  const int64_t bh = wg / nqb, h = bh % p.H, b = bh / p.H;
-  const int tid = threadIdx.x, l = tid & 63, lr = l & 15, g4 = l >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  typedef const __attribute__((address_space(4))) int32_t *list_ptr;
-  const list_ptr list = (list_ptr)(dense ? nullptr : p.idx + (bh * p.nqb + qb) * p.idx_w);
-  const uint16_t *qsrc = sp ? p.q2 + b * p.q2_sb + h * p.q2_sh : p.q + b * p.q_sb + h * p.q_sh;
-  const int64_t q_st = sp ? p.q2_st : p.q_st, nq = sp ? p.nq2 : p.nq;
-  const int64_t row0 = static_cast<int64_t>(qb) * kBlockQ + w * 32;
-  const uint16_t *kbase = p.k + b * p.k_sb + h * p.k_sh;
-  const uint16_t *vbase = p.vt + bh * p.nkb * kTile;
-  typedef __attribute__((address_space(3))) u32x4 *lds_ptr;
-  u32x4 qf[2][2];
-  for (int i = 0; i < 2; ++i) {
-    const int64_t qrow = row0 + 16 * i + lr;
-    for (int s = 0; s < 2; ++s)
-      qf[i][s] = qrow < nq ? *reinterpret_cast<const u32x4 *>(qsrc + qrow * q_st + 32 * s + 8 * g4) : u32x4{0, 0, 0, 0};
-  }
-  if (p.half_io)
-    for (int i = 0; i < 2; ++i)
-      for (int s = 0; s < 2; ++s) qf[i][s] = half8_to_bf16(qf[i][s]);
-  const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-  floatx4 oacc[2][4], lacc[2];
-  float m[2];
-  for (int i = 0; i < 2; ++i) {
-    lacc[i] = zero4;
-    m[i] = -INFINITY;
-    for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
-  }
-  // the next block's chunks wait in registers while this one is computed
-  u32x4 kr[2], vr[2];
-  int j = 0, blk = 0;
-  auto next = [&]() -> int {  // the list's next block inside the sequence, -1 at its end
-    while (j < n) {
-      blk = dense ? j : (p.delta ? blk + list[j] : list[j]);
-      ++j;
-      if (blk >= 0 && blk < p.nkb) return blk;
-    }
-    return -1;
-  };
-  auto keys_of = [&](int at) {
-    const int64_t left = p.nk - static_cast<int64_t>(at) * kBlockK;
-    return static_cast<int>(left < kBlockK ? left : kBlockK);
-  };
-  auto load = [&](int at) {
-    const int last = keys_of(at) - 1;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int ci = tid + kThreads * u, r = ci >> 3, ch = ci & 7;
-      kr[u] = *reinterpret_cast<const u32x4 *>(
-          kbase + (static_cast<int64_t>(at) * kBlockK + (r < last ? r : last)) * p.k_st + ch * 8);
-      vr[u] = *reinterpret_cast<const u32x4 *>(vbase + static_cast<int64_t>(at) * kTile + ci * 8);
-    }
-  };
-  int nxt = next();
-  if (nxt >= 0) load(nxt);
-  while (nxt >= 0) {
-    const int lim = keys_of(nxt);
-    __syncthreads();  // the previous block's reads are done
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int ci = tid + kThreads * u;
-      const int at = ((ci & ~7) | ((ci & 7) ^ swz(ci >> 3))) * 16;
-      *reinterpret_cast<lds_ptr>(lds0 + at) = kr[u];
-      *reinterpret_cast<lds_ptr>(lds0 + kTile * 2 + at) = vr[u];
-    }
-    nxt = next();
-    if (nxt >= 0) load(nxt);
-    __syncthreads();
-    floatx4 S[2][4];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int row = 32 * (kt >> 1) + 8 * (kt & 1) + 16 * (lr >> 3) + (lr & 7);
-        const u32x4 a = *reinterpret_cast<lds_ptr>(lds0 + row * 128 + ((4 * s + g4) ^ swz(row)) * 16);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) S[i][kt] = mfma16(a, qf[i][s], s == 0 ? zero4 : S[i][kt]);
-      }
-    u32x4 pb[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kk = 32 * (kt >> 1) + 8 * (kt & 1) + 16 * (g4 >> 1) + 4 * (g4 & 1) + r;
-          S[i][kt][r] = kk < lim ? S[i][kt][r] : -INFINITY;
-          mx = fmaxf(mx, S[i][kt][r]);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[i], mx * p.c);
-      const float alpha = mn == m[i] ? 1.f : __builtin_amdgcn_exp2f(m[i] - mn);
-      const float off = mn == -INFINITY ? 0.f : mn;
-      m[i] = mn;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lacc[i][r] *= alpha;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) oacc[i][t][r] *= alpha;
-      }
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int kt = 2 * s + (e >> 1), r = 2 * (e & 1);
-          pb[i][s][e] = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(S[i][kt][r], p.c, -off)),
-                                    __builtin_amdgcn_exp2f(fmaf(S[i][kt][r + 1], p.c, -off)));
-        }
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) lacc[i] = mfma16(ones, pb[i][s], lacc[i]);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int row = 16 * t + lr;
-        const u32x4 a = *reinterpret_cast<lds_ptr>(lds0 + kTile * 2 + row * 128 + ((4 * s + g4) ^ swz(row)) * 16);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) oacc[i][t] = mfma16(a, pb[i][s], oacc[i][t]);
-      }
-    }
-  }
-  store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
 }
 
 // kDense: every key block instead of a list. kUnit: c = 1 (sm_scale = ln 2:
@@ -371,9 +224,18 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const int64_t bh = unit / nqb;
   const int64_t h = bh % p.H;
   const int64_t b = bh / p.H;
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform
-  const int l = tid & 63, lr = l & 15, g4 = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave index, uniform
+  // What depends on the lane alone is formed again after the walk instead of
+  // kept through it, where every register is taken.
+  int tid, lr, g4;
+  auto lanes = [&]() __attribute__((always_inline)) {
+    int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(l));
+    tid = w * kWave + l;
+    lr = l & 15;
+    g4 = l >> 4;
+  };
+  lanes();
 
   int n;
   const int32_t *list = nullptr;
@@ -428,10 +290,8 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const int nk32 = static_cast<int>(p.nk);
   const int nkb32 = static_cast<int>(p.nkb);
   const int partial = (nk32 % kBlockK) ? nkb32 - 1 : -1;  // the partial last block, if any
-  const int r0 = tid >> 3;
-  const int kc = ((tid & 7) ^ swz_k(r0)) * 8;
-  const uint32_t koff = static_cast<uint32_t>((static_cast<int64_t>(r0) * p.k_st + kc) * 2);
-  const uint32_t voff = static_cast<uint32_t>((r0 * kHeadDim + ((tid & 7) ^ swz(r0)) * 8) * 2);
+  int r0, kc;
+  uint32_t koff, voff;
   const uint32_t lds0 = lds_addr32(smem[0][0]);
   // K and Vt of block blk -> LDS buffer buf. Blocks outside [0, nkb) load
   // block 0 (the second walk masks them); rows of the partial block past the
@@ -480,13 +340,15 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
     }
-    int lrow = lr;
-    asm volatile("" : "+v"(lrow));  // the addresses are formed again instead of kept for a second walk
-    const int krow = 16 * (lrow >> 3) + (lrow & 7);
+    r0 = tid >> 3;
+    kc = ((tid & 7) ^ swz_k(r0)) * 8;
+    koff = static_cast<uint32_t>((static_cast<int64_t>(r0) * p.k_st + kc) * 2);
+    voff = static_cast<uint32_t>((r0 * kHeadDim + ((tid & 7) ^ swz(r0)) * 8) * 2);
+    const int krow = 16 * (lr >> 3) + (lr & 7);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       ka_addr[s] = lds0 + krow * 128 + ((4 * s + g4) ^ swz_k(krow)) * 16;
-      va_addr[s] = lds0 + kTile * 2 + lrow * 128 + ((4 * s + g4) ^ swz(lrow)) * 16;
+      va_addr[s] = lds0 + kTile * 2 + lr * 128 + ((4 * s + g4) ^ swz(lr)) * 16;
     }
   };
   start();
@@ -715,84 +577,78 @@ void bsattn_fwd_kernel(const AttnParams p) {
 
   __syncthreads();  // every wave is done with the tiles and with redo
   if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0)) {
-    if (kSplit && sp) {  // combine_kernel walks the rows again
-      if (tid < kBlockQ) p.part[wg * (kBlockQ * (kHeadDim + 1)) + kBlockQ * kHeadDim + tid] = -INFINITY;
-      return;
-    }
     // again from the first block, with the queries still in registers: nothing
     // is stored before, so the output may lie on the queries' storage
-    if (idle) {
+    lanes();
+    start();
+    if (idle)
       walk(std::true_type{}, std::true_type{});
-    } else {
-      start();
+    else
       walk(std::false_type{}, std::true_type{});
-    }
   }
+  lanes();
   if (kSplit && sp) {
     float *part = p.part + wg * (kBlockQ * (kHeadDim + 1));
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = w * 32 + 16 * i + lr;
+      const float ltot = lacc[i][0];
+      const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) *reinterpret_cast<floatx4 *>(part + r * kHeadDim + 16 * t + 4 * g4) = oacc[i][t];
-      if (g4 == 0) part[kBlockQ * kHeadDim + r] = lacc[i][0];
+      for (int t = 0; t < 4; ++t)
+        *reinterpret_cast<floatx4 *>(part + r * kHeadDim + 16 * t + 4 * g4) =
+            floatx4{oacc[i][t][0] * inv, oacc[i][t][1] * inv, oacc[i][t][2] * inv, oacc[i][t][3] * inv};
+      if (g4 == 0) part[kBlockQ * kHeadDim + r] = m[i] + __builtin_amdgcn_logf(ltot);  // -inf for a sum of 0
     }
   } else {
     store_rows(p, sp, b, h, row0, nq, lr, g4, oacc, lacc);
   }
 }
 
-// Results of split special queries: the partial sums in split order, normalised
-// (thread: row tid / 2, 32 features). Rows that any part found out of range
-// are walked again, every key, with the running maximum.
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+// Results of split special queries: the parts' outputs in split order, each
+// weighted with its row sum (thread: row tid / 2, 32 features). The parts' sums
+// come as logarithms, so parts of any exponent offset meet here.
+__global__ __launch_bounds__(kThreads)
 void combine_kernel(const AttnParams p) {
-  __shared__ __attribute__((aligned(16))) uint16_t tiles[2][kTile];
   const int64_t unit = blockIdx.x;
   const int64_t bh = unit / p.nq2b, h = bh % p.H, b = bh / p.H;
   const int r = threadIdx.x >> 1, d0 = (threadIdx.x & 1) * 32;
   const int64_t qrow = (unit % p.nq2b) * kBlockQ + r;
+  if (qrow >= p.nq2) return;
+  constexpr int64_t kPart = kBlockQ * (kHeadDim + 1);
+  const float *part = p.part + unit * p.nsplit * kPart;
+  float weight[kMaxSplit], top = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < kMaxSplit; ++s)  // all loads in flight at once
+    weight[s] = s < p.nsplit ? part[s * kPart + kBlockQ * kHeadDim + r] : -INFINITY;
+#pragma unroll
+  for (int s = 0; s < kMaxSplit; ++s) top = fmaxf(top, weight[s]);
+  if (top == -INFINITY) top = 0.f;  // no part has a probability: weights 0
   floatx4 acc[8];
   float l = 0.f;
 #pragma unroll
   for (int c = 0; c < 8; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (qrow < p.nq2) {
-    for (int s = 0; s < p.nsplit; ++s) {
-      const float *part = p.part + (unit * p.nsplit + s) * (kBlockQ * (kHeadDim + 1));
-      l += part[kBlockQ * kHeadDim + r];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const floatx4 o = *reinterpret_cast<const floatx4 *>(part + r * kHeadDim + d0 + 4 * c);
+  for (int s = 0; s < kMaxSplit; ++s) {
+    if (s >= p.nsplit) break;
+    weight[s] = __builtin_amdgcn_exp2f(weight[s] - top);
+    l += weight[s];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[c][e] += o[e];
-      }
+    for (int c = 0; c < 8; ++c) {
+      const floatx4 o = *reinterpret_cast<const floatx4 *>(part + s * kPart + r * kHeadDim + d0 + 4 * c);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[c][e] = fmaf(weight[s], o[e], acc[c][e]);
     }
   }
-  // out of range, marked -inf by a part (weights are never negative), or a sum
-  // of finite parts past the float range
-  bool bad = __float_as_uint(l) - kLowBits > kHighBits - kLowBits;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t *optr = p.o2 + b * p.o2_sb + h * p.o2_sh +
+                   (p.tok_p > 0 ? (qrow / p.tok_s) * p.tok_p + qrow % p.tok_s : qrow) * p.o2_st + d0;
 #pragma unroll
-  for (int c = 0; c < 8; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bad |= (__float_as_uint(acc[c][e]) & 0x7fffffffu) >= 0x7f800000u;
-  bad = bad && qrow < p.nq2;
-  // before the stores, as in bsattn_fwd_kernel
-  if (__syncthreads_or(bad)) {
-    bsattn_online(reinterpret_cast<const AttnParams *>((const void *)__builtin_amdgcn_kernarg_segment_ptr()),
-                  lds_addr32(tiles), false, static_cast<int>(unit), static_cast<int>(p.nkb));
-    return;
-  }
-  if (qrow < p.nq2) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    uint16_t *optr = p.o2 + b * p.o2_sb + h * p.o2_sh +
-                     (p.tok_p > 0 ? (qrow / p.tok_s) * p.tok_p + qrow % p.tok_s : qrow) * p.o2_st + d0;
-#pragma unroll
-    for (int c = 0; c < 8; c += 2) {
-      const u32x4 v = {pack_bf16x2(acc[c][0] * inv, acc[c][1] * inv), pack_bf16x2(acc[c][2] * inv, acc[c][3] * inv),
-                       pack_bf16x2(acc[c + 1][0] * inv, acc[c + 1][1] * inv),
-                       pack_bf16x2(acc[c + 1][2] * inv, acc[c + 1][3] * inv)};
-      *reinterpret_cast<u32x4 *>(optr + 4 * c) = v;
-    }
+  for (int c = 0; c < 8; c += 2) {
+    const u32x4 v = {pack_bf16x2(acc[c][0] * inv, acc[c][1] * inv), pack_bf16x2(acc[c][2] * inv, acc[c][3] * inv),
+                     pack_bf16x2(acc[c + 1][0] * inv, acc[c + 1][1] * inv),
+                     pack_bf16x2(acc[c + 1][2] * inv, acc[c + 1][3] * inv)};
+    *reinterpret_cast<u32x4 *>(optr + 4 * c) = v;
   }
 }
 
@@ -1116,7 +972,7 @@ int64_t special_splits(int64_t num_wg, int64_t nkb, int64_t index_w) {
   const int64_t busy = index_w * (num_wg > 1024 ? num_wg : 1024) / 1024;
   int64_t n = busy > 0 ? (nkb + busy / 2) / busy : 1;
   if (n > nkb / 32) n = nkb / 32;
-  return n < 1 ? 1 : (n > 8 ? 8 : n);
+  return n < 1 ? 1 : (n > kMaxSplit ? kMaxSplit : n);
 }
 
 // Special-token queries of vasc_global_attn_fwd (absent: q2 == NULL).
