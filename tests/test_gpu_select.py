@@ -350,6 +350,47 @@ def test_cdf_counts_at_the_edges_of_the_row_kernels(K):
         assert np.array_equal(base.cpu().numpy(), n + (~last_in & (n < K))), (K, thr)
 
 
+@pytest.mark.parametrize("K", [65, 130, 256, 300, 577, 1036, 1089, 1600, 2048])
+def test_cdf_counts_of_clustered_rows(K):
+    """Rows whose values crowd a small part of their range, so that equal-width
+    buckets over it overflow: near-uniform probabilities beside a few large ones
+    (attention sinks) or one, two crowds far apart, signed scores, a crowd of equal
+    values with and without near neighbours, a crowd inside a crowd, infinities.
+    Counts bit-exact with the oracle."""
+    from vasc_amd import ops
+    rng = np.random.default_rng(1700 + K)
+
+    def soft(x):
+        e = np.exp(x - x.max())
+        return e / e.sum()
+    rows = []
+    for width in (0.01, 0.2, 1.0):
+        x = rng.standard_normal(K) * width
+        sinks, one = x.copy(), x.copy()
+        sinks[:4] += 5.0
+        one[3] += 8.0
+        rows += [soft(sinks), soft(one), soft(x + 6.0 * (rng.random(K) < 0.5)), x / K]
+    tied = soft(rng.standard_normal(K))
+    tied[: K * 3 // 4] = tied[0]
+    near = tied.copy()
+    near[K // 3] = np.nextafter(np.float32(tied[0]), np.float32(1))
+    nested = np.where(rng.random(K) < 0.5, 1.0 + 1e-6 * rng.random(K), 1.0 + 0.01 * rng.random(K)) / K
+    nested[0] = 0.5
+    inf = tied.copy()
+    inf[1::7] = np.inf
+    low = soft(rng.standard_normal(K))
+    low[::2] = -np.finfo(np.float32).max
+    rows += [tied, near, nested, inf, low, -tied]
+    score = np.ascontiguousarray(np.stack(rows).astype(np.float32).reshape(1, 1, -1, K))
+    s = torch.from_numpy(score).cuda()
+    for thr in (0.3, 0.9):
+        cnt, base = ops.cdf_counts(s, thr, force_last=True, want_base=True)
+        n = OS.cdf_counts(score, thr)
+        assert np.array_equal(cnt.cpu().numpy(), n), (K, thr)
+        last_in = OS.select_top(score, n)[..., K - 1]
+        assert np.array_equal(base.cpu().numpy(), n + (~last_in & (n < K))), (K, thr)
+
+
 def test_cdf_counts_c5_rows_bit_exact():
     """C5's 4096-block rows (pooled softmax of near-uniform logits), 64 rows
     at the two benchmark thresholds."""

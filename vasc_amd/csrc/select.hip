@@ -191,12 +191,15 @@ __global__ __launch_bounds__(256) void cdf_count_kernel(const float *score, int6
 // The same count for rows of up to 2048 key blocks, one wave per row (EPT keys
 // a lane). Bound by instruction issue: about 3500 VALU and 1600 SALU
 // instructions a row of 1036 blocks, half of them in the sort.
-//   sort  1024 buckets of equal key width over the positive keys' range
-//         (counting pass, scan, scatter), then each key's place among its
-//         bucket's few keys. The last bucket takes the keys <= +0, which need no
-//         order while they are all zeros. A row with a bucket above kBigBucket
-//         keys (infinities beside probabilities, planted ties) goes through a
-//         bitonic network instead.
+//   sort  1024 buckets of equal key width over the keys' range (counting pass,
+//         scan, scatter), then each key's place among its bucket's few keys. In a
+//         row without negative values the range is that of the positive keys, and
+//         the last bucket takes the zeros, which need no order. A row with a
+//         bucket above kBigBucket keys (near-equal values beside a few far larger
+//         ones, many equal values, signed values, infinities) is grouped once
+//         more, by the place interpolated in its first bucket: 1023 buckets of about
+//         equal population, each put in order by one lane, or by a bitonic network
+//         where it holds more than kBigBucket keys that are not all equal.
 //   walk  the float32 running sum S of the sorted values is sequential, but
 //         while it stays in one binade [2^e, 2^(e+1)) every addend x rounds to a
 //         multiple of 2^(e-23) by itself, unless x lies half way between two (a
@@ -206,11 +209,24 @@ __global__ __launch_bounds__(256) void cdf_count_kernel(const float *score, int6
 //         The first stretch that holds a tie or a value that is not finite and
 //         non-negative, or ends past the binade or past T, is added one by one;
 //         the scan then resumes behind it.
-// Against the radix kernel below: 1036 blocks x 8288 rows 164 -> 97 us, 1024
-// blocks x 8192 rows 102-135 -> 74-94 us; at 4096 blocks, where a row needs
-// four waves, this scheme took 1.8-2.3 ms against 1.2-1.6, so the longer rows
-// stay there.
-constexpr int kCdfBins = 1024, kBigBucket = 48;
+// us at threshold 0.9 for 16 heads of K x K / 2 blocks: the radix kernel below
+// with 1 to 8 keys a thread, this kernel with a whole-row bitonic network after
+// the first grouping, and as it is:
+//   K                                 521         1036          1600          2048
+//   softmax of N(0, 1)            68  37  38  166  95  88  257 228 226  350 339 325
+//   logits in steps of 1/16       66 109  51  168 454  95  260 783 230  368 982 316
+//   N(0, 0.2), four sinks         68  38  37  169 201 104  276 557 291  399 973 414
+//   N(0, 0.05), one large         63 106  49  165 446 105  262 757 281  373 952 394
+// Crowds of nearly equal values inside a crowd still cost up to 4 times the
+// radix kernel. At 4096 blocks, where a row needs four waves, the scheme took
+// 1.8-2.3 ms against 1.2-1.6, so the longer rows stay there. Instances of 4, 9,
+// 17 and 32 keys a lane: 47, 62, 89 and 133 VGPRs, so 8, 7, 5 and 3 waves a SIMD;
+// 9 and 17 rather than 8 and 16 because whole frames of a power of two in number
+// end a little past a power of two of blocks (1150 blocks, the 32-key instance:
+// 182 -> 137 us).
+// kBigBucket: a normal row's largest first bucket holds up to 16 keys at 1036
+// blocks, 29 at 2048.
+constexpr int kCdfBins = 1024, kBigBucket = 32;
 // Exponent distance of S from a stretch's largest value below which the
 // stretch is added one by one at once: the chance of a tie in it is about
 // kC 2^-distance.
@@ -222,10 +238,8 @@ __global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, 
   constexpr int kRow = 64 * EPT;
   constexpr int kC = EPT | 1;          // values per stretch (odd: the lanes' reads spread over the banks)
   constexpr int kOwn = kCdfBins / 64;
-  // the row, grouped and then sorted in place, and the bins; the bitonic
-  // network takes both: the power of two above K fits (K <= kRow)
+  // the row, grouped and then sorted in place, and the bins
   __shared__ __attribute__((aligned(16))) uint32_t buf[kRow + kCdfBins + 4];
-  static_assert(kRow + kCdfBins >= 2048 || kRow <= 1024, "room for the network");
   uint32_t *bins = buf + kRow;
   const int64_t row = blockIdx.x;
   const int lane = threadIdx.x;
@@ -258,26 +272,27 @@ __global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, 
   kpos = __builtin_amdgcn_readfirstlane(kpos);
   kmax = __builtin_amdgcn_readfirstlane(kmax);
 
-  // bucket of a key: 0 the largest; positive keys in [0, kCdfBins - 1), the others in the last
-  const uint32_t range = kmax > kpos ? kmax - kpos : 0u;
+  // bucket of a key: 0 the largest; keys from kfloor on in [0, kLast), zeros below it in kLast
+  constexpr uint32_t kLast = kCdfBins - 1;
+  const uint32_t kfloor = kmin < kZero ? kmin : kpos;
+  const uint32_t range = kmax > kfloor ? kmax - kfloor : 0u;
   int sh = range ? 32 - __builtin_clz(range) - 10 : 0;  // (range >> sh) < 1024
   sh = sh > 0 ? sh : 0;
-  if ((range >> sh) >= static_cast<uint32_t>(kCdfBins - 1)) ++sh;
-  auto bucket = [&](uint32_t k) { return k > kZero ? (kmax - k) >> sh : static_cast<uint32_t>(kCdfBins - 1); };
+  if ((range >> sh) >= kLast) ++sh;
+  auto bucket = [&](uint32_t k) { return k >= kfloor ? (kmax - k) >> sh : kLast; };
   __syncthreads();
   uint32_t slot[EPT];
 #pragma unroll
   for (int m = 0; m < EPT; ++m) slot[m] = lane + 64 * m < K ? atomicAdd(&bins[bucket(key[m])], 1u) : 0u;
   __syncthreads();
   // exclusive scan, kOwn bins a thread; the largest bucket that needs an order
-  // (a bucket one key wide does not, nor does the last one while it holds zeros only)
-  const bool negative = kmin < kZero;
+  // (a bucket one key wide does not, nor do the zeros of the last one)
   uint32_t own[kOwn], sum = 0u, big = 0u;
 #pragma unroll
   for (int b = 0; b < kOwn; ++b) {
     own[b] = bins[lane * kOwn + b];
     sum += own[b];
-    if (lane == 63 && b == kOwn - 1 ? negative : sh > 0) big = max(big, own[b]);
+    if (sh > 0 && !(lane == 63 && b == kOwn - 1)) big = max(big, own[b]);
   }
   uint32_t before = sum;
 #pragma unroll
@@ -309,7 +324,7 @@ __global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, 
       const uint32_t k = buf[pos];
       const uint32_t b = bucket(k), lo = bins[b], hi = bins[b + 1];
       uint32_t at = pos;
-      if (hi - lo > 1 && (b == kCdfBins - 1 ? negative : sh > 0)) {
+      if (hi - lo > 1 && b != kLast && sh > 0) {
         at = lo;
         for (uint32_t q = lo; q < hi; ++q) at += buf[q] > (q < pos ? k - 1u : k) ? 1u : 0u;  // equal keys as they lie
       }
@@ -321,24 +336,119 @@ __global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, 
     for (int m = 0; m < EPT; ++m)
       if (lane + 64 * m < K) fin[slot[m]] = key_value(key[m]);
   } else {
-    int n2 = 64;
-    while (n2 < K) n2 <<= 1;
+    // the bins' words take the first buckets' starts and the new buckets'
+    // counters, 16 bits each
+    uint16_t *first = reinterpret_cast<uint16_t *>(bins);
+    uint32_t *count = bins + kCdfBins / 2 + 2;
+    const uint16_t *end = reinterpret_cast<const uint16_t *>(count);
+    uint32_t start[kOwn];
 #pragma unroll
-    for (int m = 0; m < EPT; ++m)
-      if (lane + 64 * m < K) buf[lane + 64 * m] = key[m];
-    for (int k = K + lane; k < n2; k += 64) buf[k] = 0u;
-    for (int size = 2; size <= n2; size <<= 1) {
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        __syncthreads();
-        for (int t = lane; t < (n2 >> 1); t += 64) {
-          const int a = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), b = a + stride;  // stride: a power of two
-          const uint32_t x = buf[a], y = buf[b];
-          const bool desc = (a & size) == 0;
-          if (desc ? x < y : x > y) {
-            buf[a] = y;
-            buf[b] = x;
+    for (int b = 0; b < kOwn; ++b) start[b] = bins[lane * kOwn + b];
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < kOwn; b += 2) {
+      bins[(lane * kOwn + b) / 2] = start[b] | start[b + 1] << 16;
+      count[(lane * kOwn + b) / 2] = 0u;
+    }
+    if (lane == 0) first[kCdfBins] = static_cast<uint16_t>(K);
+    __syncthreads();
+    const float scale = static_cast<float>(kLast) / static_cast<float>(K);  // places to buckets: below kLast
+    auto place_bucket = [&](uint32_t k) {
+      const uint32_t b = bucket(k);
+      if (b == kLast) return kLast;
+      const uint32_t lo = first[b], c = first[b + 1] - lo;
+      // (kmax - k) << (32 - sh) is the place in the bucket, of 2^32 (sh > 0 here)
+      return static_cast<uint32_t>(static_cast<float>(lo + __umulhi((kmax - k) << (32 - sh), c)) * scale);
+    };
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+      if (lane + 64 * m >= K) break;
+      const uint32_t b = place_bucket(key[m]);
+      atomicAdd(&count[b >> 1], 1u << (16 * (b & 1)));
+    }
+    __syncthreads();
+    uint32_t mine = 0u;
+#pragma unroll
+    for (int b = 0; b < kOwn / 2; ++b) {
+      start[b] = count[lane * (kOwn / 2) + b];
+      mine += (start[b] & 0xffffu) + (start[b] >> 16);
+    }
+    uint32_t at = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t t = static_cast<uint32_t>(__shfl_up(static_cast<int>(at), o));
+      if (lane >= o) at += t;
+    }
+    at -= mine;
+#pragma unroll
+    for (int b = 0; b < kOwn / 2; ++b) {
+      const uint32_t even = start[b] & 0xffffu;
+      count[lane * (kOwn / 2) + b] = at | (at + even) << 16;
+      at += even + (start[b] >> 16);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {  // a counter ends as its bucket's end
+      if (lane + 64 * m >= K) break;
+      asm volatile("" : "+v"(key[m]));  // its bucket is formed again instead of kept
+      const uint32_t b = place_bucket(key[m]);
+      buf[atomicAdd(&count[b >> 1], 1u << (16 * (b & 1))) >> (16 * (b & 1)) & 0xffffu] = key[m];
+    }
+    __syncthreads();
+    // which buckets need an order: those whose keys are not all equal (bit 15 of the end)
+    constexpr uint32_t kMixed = 0x8000u;
+    auto span = [&](uint32_t b, uint32_t &lo) {
+      lo = b ? end[b - 1] & (kMixed - 1u) : 0u;
+      return static_cast<uint32_t>(end[b]);
+    };
+#pragma unroll 4
+    for (int k = lane; k < K; k += 64) {
+      const uint32_t x = buf[k], b = place_bucket(x);
+      uint32_t lo;
+      span(b, lo);
+      if (x != buf[lo]) atomicOr(&count[b >> 1], kMixed << (16 * (b & 1)));
+    }
+    __syncthreads();
+    for (uint32_t b0 = 0; b0 <= kLast; b0 += 64) {
+      uint32_t lo, hi = span(b0 + lane, lo);
+      const bool mixed = (hi & kMixed) != 0;
+      hi &= kMixed - 1u;
+      const bool large = mixed && hi - lo > kBigBucket;
+      if (mixed && !large) {  // one lane's insertion sort
+        for (uint32_t q = lo + 1; q < hi; ++q) {
+          const uint32_t x = buf[q];
+          uint32_t r = q;
+          for (; r > lo && buf[r - 1] < x; --r) buf[r] = buf[r - 1];
+          buf[r] = x;
+        }
+      }
+      for (uint64_t todo = __builtin_amdgcn_ballot_w64(large); todo != 0; todo &= todo - 1) {
+        // the whole wave's bitonic network over the bucket; every exchange moves
+        // the larger key down, so that places past its end need no padding
+        const int owner = __builtin_ctzll(todo);
+        uint32_t *part = buf + __builtin_amdgcn_readlane(static_cast<int>(lo), owner);
+        const uint32_t n = __builtin_amdgcn_readlane(static_cast<int>(hi - lo), owner);
+        auto exchange = [&](uint32_t i, uint32_t j) {
+          if (j >= n) return;
+          const uint32_t x = part[i], y = part[j];
+          if (x < y) {
+            part[i] = y;
+            part[j] = x;
+          }
+        };
+        for (uint32_t half = 1; half < n; half <<= 1) {
+          __syncthreads();
+          for (uint32_t t = lane; t < n; t += 64) {  // sorted halves: mirrored pairs, then shrinking strides
+            const uint32_t i = t & (2 * half - 1);
+            if (i < half) exchange(t, t + 2 * (half - i) - 1);
+          }
+          for (uint32_t stride = half >> 1; stride > 0; stride >>= 1) {
+            __syncthreads();
+            for (uint32_t t = lane; t < n; t += 64)
+              if (!(t & stride)) exchange(t, t + stride);
           }
         }
+        __syncthreads();
       }
     }
     __syncthreads();
