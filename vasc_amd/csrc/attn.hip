@@ -37,8 +37,10 @@
 //    block cost 2 % of the launch. Both walks take Q from the registers and
 //    only the last one stores, so the output may lie on Q's storage. Over 33312
 //    keys, 16 heads, 132 blocks a row, q and k of std 1 / 4 / 8 take 1.06 /
-//    1.15 / 1.11 ms (offset moved per block in the first walk: 1.16 / 1.19 /
-//    1.58; second walk with a new maximum each block: 1.06 / 1.88 / 1.48).
+//    1.18 / 1.12 ms (offset moved per block in the first walk: 1.17 / 1.20 /
+//    1.60; second walk with a new maximum each block: 1.06 / 1.88 / 1.48). The
+//    first walk ends a block after the look that failed: leaving at once, by a
+//    break or an empty block, costs every launch 0.3 to 1 % (or spills).
 //  * Keys past the sequence end (the partial last block) read the last key's
 //    row: their V rows are zero and the ones operand is zeroed there.
 //  * K and Vt tiles arrive by LDS DMA (global_load_lds_dwordx4) into a
@@ -521,8 +523,8 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma clang loop unroll(disable)
     for (int j = 0; j < nw; ++j) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (!kOnline && j == look + 1) {
-        if (__builtin_amdgcn_readfirstlane(redo)) nw = 0;
+      if (!kOnline && __builtin_expect(j == look + 1, 0)) {
+        if (__builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
         look = 2 * look + 8;
       }
       const int lim = valid_keys(blk);
@@ -544,9 +546,9 @@ void bsattn_fwd_kernel(const AttnParams p) {
             set_ones(lim);
             out_of_list |= lim == 0;
           }
-          if (nw) compute();
+          compute();
           if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
-          if (j == look && sums_bad(look ? kLaterBits : kFirstBits)) redo = 1;
+          if (__builtin_expect(j == look, 0) && sums_bad(look ? kLaterBits : kFirstBits)) redo = 1;
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
