@@ -348,6 +348,14 @@ def test_cdf_counts_at_the_edges_of_the_row_kernels(K):
         assert np.array_equal(cnt.cpu().numpy(), n), (K, thr)
         last_in = OS.select_top(score, n)[..., K - 1]
         assert np.array_equal(base.cpu().numpy(), n + (~last_in & (n < K))), (K, thr)
+        _check_many_rows(ops, s, thr, cnt, base)
+
+
+def _check_many_rows(ops, s, thr, cnt, base):
+    """The same rows repeated until the kernel with one wave per row counts them."""
+    times = 2049 // s.shape[2] + 1
+    many, many_base = ops.cdf_counts(s.repeat(1, 1, times, 1), thr, force_last=True, want_base=True)
+    assert torch.equal(many, cnt.repeat(1, 1, times)) and torch.equal(many_base, base.repeat(1, 1, times))
 
 
 @pytest.mark.parametrize("K", [65, 130, 256, 300, 577, 1036, 1089, 1600, 2048])
@@ -389,6 +397,7 @@ def test_cdf_counts_of_clustered_rows(K):
         assert np.array_equal(cnt.cpu().numpy(), n), (K, thr)
         last_in = OS.select_top(score, n)[..., K - 1]
         assert np.array_equal(base.cpu().numpy(), n + (~last_in & (n < K))), (K, thr)
+        _check_many_rows(ops, s, thr, cnt, base)
 
 
 def test_cdf_counts_c5_rows_bit_exact():

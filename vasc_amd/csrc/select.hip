@@ -530,8 +530,9 @@ __global__ __launch_bounds__(64) void cdf_count_rows_kernel(const float *score, 
   }
 }
 
-// The same count for rows of 2049 to 4096 key blocks, with the row sorted by rocPRIM's LDS block radix sort (256
-// threads, kItems keys each; 8-bit digits, four passes over 32-bit keys)
+// The same count for rows of 2049 to 4096 key blocks, and for few shorter rows,
+// with the row sorted by rocPRIM's LDS block radix sort (256 threads, kItems
+// keys each; 8-bit digits, four passes over 32-bit keys)
 // instead of the bitonic network, which costs O(K log^2 K) compare-exchanges
 // with a barrier per stage. Keys load lane-strided (coalesced), padding keys
 // 0 sort last; after the descending sort thread t holds ranks
@@ -2807,7 +2808,17 @@ extern "C" int vasc_cdf_counts(const float *score, int64_t B, int64_t H, int64_t
   const dim3 grid(static_cast<unsigned>(B * H * Q));
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int Ki = static_cast<int>(K);
-  if (K <= 64 * 32) {
+  // One wave per row needs rows for every SIMD (1024): below that the radix kernel's
+  // four waves end a row sooner. us for 65 to 576 blocks, mean of near-uniform,
+  // N(0, 1), quantised and sink rows, radix and rows kernel: 520 rows of 130 blocks
+  // 7.7 and 9.9, 1040 rows 9.6 and 10.5, 2080 rows 13.7 and 11.6; 1024 rows of 256
+  // blocks 10.3 and 14.0, 2048 13.8 and 14.5, 4096 23.2 and 17.8; 600 rows of 300
+  // blocks 11.3 and 14.6, 1800 17.5 and 16.0; 700 rows of 700 blocks 17.9 and 24.3,
+  // 1400 25.1 and 25.2, 2800 37.9 and 27.8. Up to 64 blocks the rows kernel leads at
+  // any number (33 blocks, 544 rows: 7.0 and 5.8).
+  const int64_t rows = B * H * Q;
+  const bool few = K > 64 && rows <= (K > 128 && K <= 256 ? 2048 : 1023);
+  if (K <= 64 * 32 && !few) {
     auto kern = K <= 64 * 4    ? cdf_count_rows_kernel<4>
                 : K <= 64 * 9  ? cdf_count_rows_kernel<9>
                 : K <= 64 * 17 ? cdf_count_rows_kernel<17>
@@ -2817,8 +2828,13 @@ extern "C" int vasc_cdf_counts(const float *score, int64_t B, int64_t H, int64_t
     return check_launch("vasc_cdf_counts");
   }
   if (K <= 256 * 16) {
-    hipLaunchKernelGGL(cdf_count_radix_kernel<16>, grid, dim3(256), 0, st, score, H, Q, Ki, thresholds, min_count,
-                       force_last, count_out, base_out);
+    auto kern = K <= 256    ? cdf_count_radix_kernel<1>
+                : K <= 512  ? cdf_count_radix_kernel<2>
+                : K <= 1024 ? cdf_count_radix_kernel<4>
+                : K <= 2048 ? cdf_count_radix_kernel<8>
+                            : cdf_count_radix_kernel<16>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, score, H, Q, Ki, thresholds, min_count, force_last, count_out,
+                       base_out);
     return check_launch("vasc_cdf_counts");
   }
   int n2 = 64;
