@@ -10,11 +10,12 @@
 //  * 4 waves x 32 query rows (two tiles of 16). S^T = K Q^T on
 //    v_mfma_f32_16x16x32_bf16, so a lane owns one query row of each tile
 //    (lane % 16) and 16 of the 64 keys of a block.
-//  * The kernel runs at the card's power limit, so the clock follows what a
-//    block costs in energy: with random bf16 operands the 16x16x32 product
-//    sustains 2.23 PFLOP/s and the 32x32x16 one 1.89 (accumulators move half
-//    the register bytes per product). The change of shape took a launch over
-//    33312 keys, 16 heads and 132 blocks a row from 1.13 to 1.02 ms.
+//  * The clock falls to a mean of 1.67 GHz of 2.4 under this kernel (counters
+//    of a launch over 33312 keys, 16 heads and 132 blocks a row), so what a
+//    block costs in energy counts. On random operands the 16x16x32 product
+//    sustains 1.59 PFLOP/s at 2.06 GHz and the 32x32x16 one 1.50 at 1.89
+//    (accumulators move half the register bytes per product). The change of
+//    shape took that launch from 1.13 to 1.02 ms.
 //  * O^T = Vt P^T on the same MFMA, so P feeds the B operand straight from
 //    the S^T accumulators. Vt comes from vasc_pack_v with its keys permuted;
 //    row i of S^T tile u of a 32-key group is key 8 u + 16 (i / 8) + i % 8 of
@@ -24,9 +25,10 @@
 //    beside 16 MFMAs and the exponentials cost a wave-block 350 cycles, the
 //    products 47 (probe without memory, four waves per SIMD).
 //  * The kernel is held to 128 VGPRs so four waves share each SIMD: MFMAs of
-//    one wave overlap the exponentials of the others (about 770 cycles per
-//    wave-block: 576 of MFMA, 450 of VALU). Two waves of 64 rows per SIMD
-//    halve the LDS reads but took 980 cycles (exposed latencies).
+//    one wave overlap the exponentials of the others. In the launch above a
+//    wave-block takes 943 cycles, 576 of them MFMA; in a probe without memory
+//    770, where two waves of 64 rows per SIMD, which halve the LDS reads, took
+//    980 (exposed latencies).
 //  * Softmax is invariant to the exponent offset, which only has to keep the
 //    probabilities inside fp32/bf16 range. The walk uses offset 0:
 //    P = exp2(c S) on the exact fp32 logits, no max, no rescale, no branch.
