@@ -541,7 +541,8 @@ int vasc_block_sparse_attn_f16_fwd(const uint16_t *q, int64_t q_sb, int64_t q_sh
 
 /* vasc_pack_global with q_patch and q_special written as
  * bf16(q * q_scale), one rounding after the norm and the rotary embedding
- * (q_scale > 0; the pooled means stay those of the unscaled bf16 rows).
+ * (q_scale > 0; the pooled means stay those of the unscaled bf16 rows). Rows
+ * without either are bf16 as read: there the product is a rounding more.
  * With q_scale = log2(e) * sm_scale the attention entry points take
  * sm_scale = ln 2, and the list-driven ones then need no product per score. */
 int vasc_pack_global_scaled(const uint16_t *q, int64_t q_sb, int64_t q_st, int64_t q_sh,

@@ -590,3 +590,23 @@ def test_half_inputs_equal_their_bf16_casts(nq, nk, strided):
     ref = ops.block_sparse_attn(qc, kc, vt, idx, cnt)
     assert torch.equal(ops.block_sparse_attn(q, kb, vt, idx, cnt), ref)
     assert torch.equal(ops.block_sparse_attn(q, kb, vt, idx, cnt, half_out=True), ref.to(torch.float16))
+
+
+@pytest.mark.parametrize("nq,nk", [(130, 193), (257, 64)])
+def test_half_inputs_in_batches(nq, nk):
+    """Two batch entries and heads in either order of strides: the float16 pooling,
+    packing and attention read every (batch, head) row of strided tensors as they
+    read contiguous ones, and as the bf16 kernels read the casts."""
+    from vasc_amd import ops
+    B, H, D = 2, 3, 64
+    q, k, v = (_rand((B, n, H, D), 95 + i).to(torch.float16).cuda().transpose(1, 2) for i, n in enumerate((nq, nk, nk)))
+    dense = [t.contiguous() for t in (q, k, v)]
+    casts = [t.to(torch.bfloat16) for t in dense]
+    for a, b, c in zip(ops.pool_qkv(q, k, v), ops.pool_qkv(*dense), ops.pool_qkv(*casts)):
+        assert torch.equal(a, b) and torch.equal(a, c)
+    kb, vt = ops.pack_kv_half(k, v)
+    assert torch.equal(kb, casts[1]) and torch.equal(vt, ops.pack_v(casts[2]))
+    idx, cnt = (torch.from_numpy(t).cuda() for t in _lists(B, H, math.ceil(nq / 128), math.ceil(nk / 64), 96, 0.6))
+    ref = ops.block_sparse_attn(casts[0], kb, vt, idx, cnt)
+    assert torch.equal(ops.block_sparse_attn(q, kb, vt, idx, cnt, half_out=True), ref.to(torch.float16))
+    _check(ref, OA.block_sparse_attention(*(t.float().cpu().numpy() for t in casts), idx.cpu().numpy(), cnt.cpu().numpy()))
