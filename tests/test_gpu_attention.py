@@ -240,6 +240,46 @@ def test_range_exit_at_every_point_of_the_walk(nblk, at, reverse, hot):
     _check(ops.dense_attn(qc, kc, vt), ref)
 
 
+@pytest.mark.parametrize("form", ["listed", "delta", "special"])
+@pytest.mark.parametrize("later", [0.0, 60.0, 200.0])
+@pytest.mark.parametrize("nblk,at", [(2, 0), (3, 0), (4, 0), (10, 8), (11, 8), (28, 24), (70, 0), (70, 56)])
+def test_walk_goes_on_with_good_sums(nblk, at, later, form):
+    """Row sums near 2^100 (block 0) or 2^110 (later blocks) after a look at them:
+    the walk is left two blocks on with sums that are good at exponent offset 0,
+    and the rest of the list, the partial last block in it, is added to them; its
+    last block lies at 2^``later``, up to a move of the offset. Special queries:
+    70 blocks go in two parts, beside a patch block of the same list."""
+    from vasc_amd import _lib, ops
+    from oracle import lut as OL
+    B, H, nq, nk, D = 1, 2, 130, 64 * nblk - 31, 64
+    q, k, v = (_rand((B, H, n, D), 33 + i) for i, n in enumerate((nq, nk, nk)))
+    level = torch.zeros(nblk)
+    level[at] = 110.0 if at else 100.0
+    if at + 2 < nblk:
+        level[-1] = later
+    q[..., 0] = 0.0
+    q[:, :, ::3, 0] = 8.0  # log2 logit: q0 * k0 / 8 * log2(e)
+    k[..., 0] = (level / math.log2(math.e)).to(torch.bfloat16).repeat_interleave(64)[:nk]
+    idx = np.ascontiguousarray(np.broadcast_to(np.arange(nblk, dtype=np.int32), (B, H, 2, nblk)))
+    cnt = np.full((B, H, 2), nblk, np.int32)
+    left = _log2_sums(q, k, idx, np.full((B, H, 2), min(at + 2, nblk), np.int32))[:, :, ::3]
+    assert (left > (104 if at else 72)).all() and (left < 119).all()
+    ref = OA.block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), idx, cnt)
+    qc, kc, vt = q.cuda(), k.cuda(), ops.pack_v(v.cuda())
+    ic, cc = torch.from_numpy(idx).cuda(), torch.from_numpy(cnt).cuda()
+    if form == "special":
+        qp, one = qc[:, :, :128], torch.ones_like(cc[:, :, :1])
+        assert (_lib.fn("vasc_global_attn_workspace_size")(B, H, 128, nq, nk, 1) > 0) == (nblk == 70)
+        _check(ops.global_attn(qp, qc, kc, vt, ic[:, :, :1, :1].contiguous(), one)[1], ref)
+    elif form == "delta":
+        lut, n = OL.encode(np.ones((B, H, 2, nblk), bool))
+        assert (n == cnt).all()
+        _check(ops.block_sparse_attn(qc, kc, vt, torch.from_numpy(lut).cuda(), cc, delta=True), ref)
+    else:
+        _check(ops.block_sparse_attn(qc, kc, vt, ic, cc), ref)
+        _check(ops.dense_attn(qc, kc, vt), ref)
+
+
 @pytest.mark.parametrize("N,P,S,H", [(1, 129, 1, 1), (3, 47, 5, 3), (2, 130, 0, 9)])
 def test_prescaled_queries_match_the_oracle(N, P, S, H):
     """Queries packed with the softmax scale: the layout differs in q only, the

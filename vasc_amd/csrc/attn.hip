@@ -35,11 +35,12 @@
 //    Where c is 1 the product goes too. A row sum outside [2^-60, 2^120]
 //    (looked at after blocks 0, 8, 24, 56, .. and at the end) sends the
 //    workgroup through a second walk, whose offset follows the row maximum and
-//    which also takes blocks outside the sequence. Checking and rescaling per
-//    block cost 2 % of the launch. Both walks take Q from the registers and
+//    which also takes blocks outside the sequence; a walk that is about to leave
+//    the range goes on in that form from where it stands. Checking and rescaling
+//    per block cost 2 % of the launch. Both walks take Q from the registers and
 //    only the last one stores, so the output may lie on Q's storage. Over 33312
-//    keys, 16 heads, 132 blocks a row, q and k of std 1 / 4 / 8 take 1.06 /
-//    1.18 / 1.12 ms (offset moved per block in the first walk: 1.17 / 1.20 /
+//    keys, 16 heads, 132 blocks a row, q and k of std 1 / 4 / 8 take 1.05 /
+//    1.15 / 1.12 ms (offset moved per block in the first walk: 1.17 / 1.20 /
 //    1.60; second walk with a new maximum each block: 1.06 / 1.88 / 1.48). The
 //    first walk ends a block after the look that failed: leaving at once, by a
 //    break or an empty block, costs every launch 0.3 to 1 % (or spills).
@@ -144,10 +145,14 @@ constexpr float kLow = 8.673617379884035e-19f;    // 2^-60
 // them. A walk whose sums will leave the range is better left early: above 2^72
 // after the first block (3.9 standard deviations, the largest of its 8192
 // scores, where the walk's largest of a million lie at 4.9 to 5.2), later above
-// 2^104. A needless second walk costs 5 to 10 %, a late one twice the time.
+// 2^104. Sums still in the range then are kept and the second form goes on from
+// them, 5 to 10 % slower a block; a walk left late starts again, at twice the time.
+// Kept against started again, std 4: 17 blocks a row 193 -> 178 us, 9 blocks
+// 19.1 -> 17.1, 34 blocks 103 -> 97 (offset moved per block: 184, 16.5, 100).
 constexpr uint32_t kHighBits = 0x7b800000u, kLaterBits = 0x73800000u, kFirstBits = 0x63800000u, kLowBits = 0x21800000u;
 // Second walk (see compute_online).
 constexpr float kRaise = 64.f, kMargin = 32.f;
+constexpr uint32_t kLeave = 1u, kRedo = 2u;
 
 constexpr int kMaxSplit = 8;  // workgroups that share a special-query block's keys
 
@@ -210,7 +215,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   constexpr int CH = 512 / kThreads;  // 16-byte chunks per thread per tile
   constexpr uint32_t kBufBytes = 2 * kTile * 2;
   __shared__ __attribute__((aligned(2 * kBufBytes))) uint16_t smem[2][2][kTile];  // [buffer][K, Vt]
-  __shared__ int redo;  // a wave's row sums left the range of offset 0
+  __shared__ uint32_t redo;  // a wave's row sums are about to leave the range of offset 0 (kLeave) or have left it (kRedo)
 
   // Workgroups [0, num_wg2_slots) take the special-token queries (every key
   // block; the slot count is rounded up to a multiple of the 8 XCDs so that
@@ -336,7 +341,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
   // K tile and row lr of the Vt tile, chunk 4 s + g4
   typedef const __attribute__((address_space(3))) u32x4 *lds_ptr;
   uint32_t ka_addr[2], va_addr[2];
-  auto start = [&]() __attribute__((always_inline)) {
+  auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       lacc[i] = zero4;
@@ -344,6 +349,8 @@ void bsattn_fwd_kernel(const AttnParams p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) oacc[i][t] = zero4;
     }
+  };
+  auto start = [&]() __attribute__((always_inline)) {
     r0 = tid >> 3;
     kc = ((tid & 7) ^ swz_k(r0)) * 8;
     koff = static_cast<uint32_t>((static_cast<int64_t>(r0) * p.k_st + kc) * 2);
@@ -355,6 +362,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
       va_addr[s] = lds0 + kTile * 2 + lr * 128 + ((4 * s + g4) ^ swz(lr)) * 16;
     }
   };
+  clear();
   start();
   auto k_op = [&](int kt, int s) {
     return *reinterpret_cast<lds_ptr>(ka_addr[s] + (32 * (kt >> 1) + 8 * (kt & 1)) * 128);
@@ -513,17 +521,21 @@ void bsattn_fwd_kernel(const AttnParams p) {
   const __attribute__((address_space(4))) int32_t *clist =
       (const __attribute__((address_space(4))) int32_t *)(list);
   bool out_of_list = false;  // a block outside the sequence was listed
+  int done = 0;              // blocks of the list that are in the sums
   // The walk: wait for a block's tiles, start the next block's DMA into the
   // other buffer, compute. kIdle: a wave without rows, which only stages its
   // share of the tiles and keeps the barriers. kOnline: the second walk.
   auto walk = [&](auto idle_wave, auto online) __attribute__((always_inline)) {
     constexpr bool kIdle = decltype(idle_wave)::value, kOnline = decltype(online)::value;
-    int blk = dense ? blk0 : clist[0];
-    int32_t e_next = dense ? 0 : clist[n > 1 ? 1 : 0];
+    const int j0 = kOnline ? done : 0;  // even: the walk is left a block after an even look
+    int blk = dense ? blk0 + j0 : clist[j0];
+    if (kOnline && !dense && p.delta)
+      for (int i = 0; i < j0; ++i) blk += clist[i];  // not kept through the first walk, which has no registers to spare
+    int32_t e_next = dense ? 0 : clist[j0 + 1 < n ? j0 + 1 : j0];
     fetch(blk, 0);
     int nw = n, look = 0;  // look: the block after which the row sums are looked at next (0, 8, 24, 56, ..)
 #pragma clang loop unroll(disable)
-    for (int j = 0; j < nw; ++j) {
+    for (int j = j0; j < nw; ++j) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       if (!kOnline && __builtin_expect(j == look + 1, 0)) {
         if (__builtin_amdgcn_readfirstlane(redo)) nw = j + 1;  // ends after this block
@@ -550,7 +562,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
           }
           compute();
           if (__builtin_expect(lim < kBlockK, 0)) sum_a[0] = sum_a[1] = ones;
-          if (__builtin_expect(j == look, 0) && sums_bad(look ? kLaterBits : kFirstBits)) redo = 1;
+          if (__builtin_expect(j == look, 0) && sums_bad(look ? kLaterBits : kFirstBits)) atomicOr(&redo, kLeave);
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -559,6 +571,7 @@ void bsattn_fwd_kernel(const AttnParams p) {
         }
       }
     }
+    done = nw;
   };
   if (n > 0) {
     if (idle) {
@@ -575,16 +588,24 @@ void bsattn_fwd_kernel(const AttnParams p) {
             const uint32_t o = __float_as_uint(oacc[i][t][r]) & 0x7fffffffu;
             top = o > top ? o : top;
           }
-      if (sums_bad(kHighBits) || __ballot(top >= 0x7f800000u) != 0 || out_of_list) redo = 1;
+      if (sums_bad(kHighBits) || __ballot(top >= 0x7f800000u) != 0 || out_of_list) atomicOr(&redo, kRedo);
     }
   }
 
   __syncthreads();  // every wave is done with the tiles and with redo
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane(redo), 0)) {
-    // again from the first block, with the queries still in registers: nothing
-    // is stored before, so the output may lie on the queries' storage
+  const uint32_t flags = __builtin_amdgcn_readfirstlane(redo);
+  const bool again = (flags & kRedo) != 0;
+  if (__builtin_expect(flags != 0, 0) && (again || done < n)) {
+    // on from where the first walk ended, its sums being good at offset 0, or
+    // again from the first block, with the queries still in registers: nothing is
+    // stored before, so the output may lie on the queries' storage
     lanes();
     start();
+    unset = again;
+    if (again) {
+      clear();
+      done = 0;
+    }
     if (idle)
       walk(std::true_type{}, std::true_type{});
     else
