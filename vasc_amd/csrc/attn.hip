@@ -986,13 +986,15 @@ struct OutTokens {
 // every key block while a patch block walks its list (index_w entries), and the
 // patch blocks keep the card (1024 resident workgroups) busy for about
 // index_w * max(1, num_wg / 1024) of these steps: the special blocks are split to
-// end with them, into parts of at least 32 key blocks. Below 64 blocks the second
-// launch and the workspace cost the host more than the split saves: at 2 frames of
-// 1041 tokens the launch fell from 29 to 24 us and the layer, bound by the host,
-// rose from 421 to 435. To the nearest part count: two parts for a walk that
-// already ends with the patch blocks cost the 32-frame layer 0.4 to 1.1%. Unsplit,
-// patch blocks alone and split, 16 heads, lists of a quarter: 56, 30 and 39 us at
-// 4 frames; 120, 89 and 97 at 8; 300, 289 and 296 at 16.
+// end with them, into parts of at least 32 key blocks. The host knows the width
+// only: counts far below it, as a cdf threshold gives, leave a walk unsplit (8
+// frames, counts a quarter of a full width: 117 us, split 98). Below 64 blocks
+// the second launch and the workspace cost the host more than the split saves: at
+// 2 frames of 1041 tokens the launch fell from 29 to 24 us and the layer, bound by
+// the host, rose from 421 to 435. To the nearest part count: two parts for a walk
+// that already ends with the patch blocks cost the 32-frame layer 0.4 to 1.1%.
+// Unsplit, patch blocks alone and split, 16 heads, lists of a quarter: 56, 30 and
+// 39 us at 4 frames; 120, 89 and 97 at 8; 300, 289 and 296 at 16.
 int64_t special_splits(int64_t num_wg, int64_t nkb, int64_t index_w) {
   const int64_t busy = index_w * (num_wg > 1024 ? num_wg : 1024) / 1024;
   int64_t n = busy > 0 ? (nkb + busy / 2) / busy : 1;
